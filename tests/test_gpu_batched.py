@@ -237,6 +237,40 @@ def test_s512_default_shape_matches_16x32(method, n):
     assert bits_equal(x_def, x_ref)
 
 
+# slices of several DPP rows (s = 512, 1024, 2048): one slice per system, the
+# largest systems of one workgroup, and the one size that keeps 32 equations
+# per lane
+@pytest.mark.parametrize("n,s", [(512, 512), (2048, 512), (16384, 512), (1024, 1024), (16384, 1024), (2048, 2048),
+                                 (16384, 2048), (32768, 2048)])
+def test_fast_ptpr_wide_slices(n, s):
+    """Fast PTPR on slices above one DPP row runs as rows of 256 equations:
+    within the fast tolerance of the oracle, as accurate as it against the
+    truth, and (up to n = 16384) the bits of s = 256 -- with a diagonal and
+    without, and with fp16 storage, a refinement step and a shared matrix."""
+    nsys = 3
+    say("wide slices", n, s)
+    a, b, c, d, xt = O.gen_batch(29, 0, nsys, n)
+    x = gpu_solve(a, b, c, d, n, s, "ptpr", "fast")
+    ref = O.solve_batch("ptpr", a, b, c, d, n, s)
+    assert per_system_rel(x, ref, n).max() <= FAST_TOL
+    assert per_system_rel(x, xt, n).max() <= max(2 * per_system_rel(ref, xt, n).max(), 1e-6)
+    na, nc, nd = O.normalize(a, b, c, d)
+    assert per_system_rel(gpu_solve(na, None, nc, nd, n, s, "ptpr", "fast"), ref, n).max() <= FAST_TOL
+    if n > 16384:
+        return
+    assert bits_equal(x, gpu_solve(a, b, c, d, n, 256, "ptpr", "fast"))
+    da, db, dc, dd = to_dev(a, b, c, d)
+    h = [v.half() for v in (da, db, dc)]
+    for kw, coef in (({}, h), ({"refine": True}, (da, db, dc)), ({"shared": True}, [v[:n] for v in (da, db, dc)])):
+        got = []
+        for sl in (s, 256):
+            dx = torch.from_numpy(ref).cuda()
+            B.solve_ex(*coef, dd, dx, n, sl, arith="fast", **kw)
+            torch.cuda.synchronize()
+            got.append(dx.cpu().numpy())
+        assert bits_equal(*got), kw
+
+
 @pytest.mark.parametrize("method", ["ptpr", "tpr"])
 def test_full_batch_4096x1024(method):
     """4096 systems x N = 1024, S = 256, generated on the GPU: exact is

@@ -135,10 +135,12 @@ def default_batched_shape(s):
 
 def fast_form(method, E, L):
     """Which fast-arithmetic stage 1 a slice shape runs: PTPR on slices of
-    one 16-lane DPP row with E >= 2 takes the two-level form (a Thomas sweep
-    in each lane, PCR across the lanes' last rows), every other shape the
-    register PCR; shapes of one form give the same bits."""
-    return "two-level" if method == "ptpr" and L == 16 and E >= 2 else "pcr"
+    one 16-lane DPP row with E >= 2, or of several such rows (16 x 32, 16 x
+    64, 32 x 64), takes the two-level form (a Thomas sweep in each lane, PCR
+    across the lanes' last rows), every other shape the register PCR; shapes
+    of one form and slice size give the same bits."""
+    rows = (L == 16 and E >= 2) or (L > 16 and E >= 16)
+    return "two-level" if method == "ptpr" and rows else "pcr"
 
 
 def batched_candidates(n, s):

@@ -127,7 +127,7 @@ hipError_t launch_variant(const BatchArgs& p, int grid, int block, size_t shmem,
 }
 
 template <int METHOD, int E, int L, int MODE>
-hipError_t launch_el(const BatchArgs& p, hipStream_t stream) {
+hipError_t launch_el_t(const BatchArgs& p, hipStream_t stream) {
     const int T = p.m * L;  // lanes per system, a power of two
     const int lg = __builtin_ctz((unsigned)T);
     const int block = T <= 64 ? kSmallBlock : T;
@@ -146,6 +146,13 @@ hipError_t launch_el(const BatchArgs& p, hipStream_t stream) {
                               : launch_variant<METHOD, E, L, MODE, 1024>(p, grid, block, shmem, lg, stream);
     if (e != hipSuccess) return e;
     return hipGetLastError();
+}
+
+template <int METHOD, int E, int L, int MODE>
+hipError_t launch_el(const BatchArgs& p, hipStream_t stream) {
+    // fast PTPR takes these shapes as rows of 16 lanes (batched_ptpr.hip)
+    if constexpr (METHOD == 0 && MODE == kFast && E == 16 && L > 16) return hipErrorInvalidValue;
+    else return launch_el_t<METHOD, E, L, MODE>(p, stream);
 }
 
 template <int METHOD, int MODE>

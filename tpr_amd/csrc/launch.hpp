@@ -61,6 +61,19 @@ constexpr bool is_default_shape(int E, int L) {
            (E == 16 && (L == 32 || L == 64)) || (E == 32 && L == 64);
 }
 
+// Fast PTPR on slices of s = 512, 1024 and 2048 (E = 16 on 32 or 64 lanes,
+// E = 32 on 64) runs as rows of 16 lanes x 16 equations: a slice's interior
+// may be eliminated in any order in fast arithmetic, and the two-level stage
+// 1 needs one Thomas sweep per lane and four DPP levels per row where the
+// register PCR across 32 or 64 lanes takes nine to eleven levels over every
+// equation, most of them through ds_bpermute (2047 x N=2048 at s = 512: 30.0
+// us that way, 15.2 this way and HBM bound; one system 8.2 against 4.5).  A
+// system must then fit one workgroup at 16 equations
+// per lane: n <= 16384 (32768 at s = 2048 keeps 32 equations per lane).
+inline bool fast_rows_16(int E, int L, int n) {
+    return ((E == 16 && (L == 32 || L == 64)) || (E == 32 && L == 64)) && n <= 16384;
+}
+
 struct BatchArgs {
     const void* a;  // float, or _Float16 when f16
     const void* b;  // may be null: unit diagonal
