@@ -14,8 +14,9 @@
 // Every call on one GPU shares that GPU's array: calls that overlap on the
 // device (different streams without ordering between them) race on it.
 // Nothing in it needs clearing by the caller: each round of the split path
-// writes every word it later reads (the one-pass form's tickets and flags are
-// zeroed by a fill kernel at the start of its round, not by hipMemsetAsync).
+// writes every word it later reads (the one-pass forms' exchange words are
+// cleared by a fill kernel at the start of their round, not by
+// hipMemsetAsync).
 #include <hip/hip_runtime.h>
 
 #include <mutex>

@@ -7,7 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "launch_serve.hpp"
-#include "split_kernels.hpp"
+#include "split_fused.hpp"
 
 namespace tprh {
 
@@ -29,6 +29,13 @@ namespace {
 template <int METHOD, int E, int L, int MODE>
 hipError_t launch_el(const ServeSplitLaunch& p, hipStream_t stream) {
     const int m = p.n / (E * L);
+    if constexpr (METHOD == 0 && MODE == kFast) {
+        // one pass (split_fused.hpp); every shape here has s >= 256
+        bool done = false;
+        const hipError_t e =
+            launch_fused<true, float, false>(TableLoc{p.sys, p.base, p.n, m}, p.n, p.nsys, stream, &done);
+        if (e != hipSuccess || done) return e;
+    }
     const int lg_m = __builtin_ctz((unsigned)m);
     static std::atomic<unsigned long long> lds_set{0};  // K2 keeps 10 rows of m floats in LDS
     hipError_t le = ensure_lds_limit(reinterpret_cast<const void*>(reduced_kernel<METHOD, TableLoc>),

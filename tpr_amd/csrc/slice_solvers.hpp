@@ -844,19 +844,27 @@ __device__ __forceinline__ void fast16_stage1(const RawPart<E>& p, bool has_b, i
     st.sR = __builtin_fmaf(q[0], st.eR, y[0]);
 }
 
-// Second half: stage 3 from x[st-1] = xprev, x[ed] = xe and the slice's
-// last row se (as the reference's stage 3 takes them).
+// Second half: every x of the lane from x[st-1] = xprev, x[ed] = xe and
+// x[ed+1] = key.
 template <int E>
-__device__ __forceinline__ void fast16_stage3(const Fast16State<E>& st, float xprev, float xe, SliceEnd se, int l,
+__device__ __forceinline__ void fast16_finish(const Fast16State<E>& st, float xprev, float xe, float key, int l,
                                               float (&X)[E]) {
-    float key = fast_rcp(se.c) * (__builtin_fmaf(-se.a, xprev, se.r) - xe);
-    if (se.c == 0.0f) key = 0.0f;
     float e = __builtin_fmaf(-st.eC, key, __builtin_fmaf(-st.eA, xprev, st.eR));
     if (l == 15) e = xe;
     const float eprev = shift_up<16, 1>(e, xprev, l);
 #pragma unroll
     for (int k = 0; k < E - 1; k++) X[k] = __builtin_fmaf(st.q[k], e, __builtin_fmaf(st.pc[k], eprev, st.y[k]));
     X[E - 1] = e;
+}
+
+// Stage 3 from xprev, xe and the slice's last row se, which gives x[ed+1] as
+// the reference's stage 3 takes it.
+template <int E>
+__device__ __forceinline__ void fast16_stage3(const Fast16State<E>& st, float xprev, float xe, SliceEnd se, int l,
+                                              float (&X)[E]) {
+    float key = fast_rcp(se.c) * (__builtin_fmaf(-se.a, xprev, se.r) - xe);
+    if (se.c == 0.0f) key = 0.0f;
+    fast16_finish<E>(st, xprev, xe, key, l, X);
 }
 
 template <int E, bool WAVE>

@@ -5,9 +5,13 @@
 //
 // The reference needs every block of a system co-resident for its grid-wide
 // barriers and limits n to s^2 (src/ptpr.cu:543,581,655).  Here a batch is
-// solved in rounds of `chunk` systems, each round in one of three forms:
+// solved in rounds of `chunk` systems, each round in one of four forms:
 //
-// Two passes (split_kernels.hpp), the library's form:
+// Fused (split_fused.hpp), the library's form for fast PTPR at s >= 256 (and
+// what split_form 2 asks for there): one pass over tiles that exchange six
+// numbers each, 65 us for 256 x N=65536.
+//
+// Two passes (split_kernels.hpp), the library's form for everything else:
 //   K1 rows_kernel   : every lane group reduces its slices and writes two
 //                      boundary rows per slice (E_st before its update, E_ed);
 //   K2 reduced_kernel: one workgroup per system applies E_st += s1 E_ed
@@ -44,12 +48,13 @@
 // the reloads it saves, which the last-level cache serves only about 1.4x
 // faster than HBM on this part.
 //
-// The library chooses two passes.  Exact answers are the same bits in every
+// Exact answers are the same bits in every
 // form (the same operations in the same order); fast answers agree within
 // rounding (the forms differ in where stage 1's end rows come from).
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "split_fused.hpp"
 #include "split_kernels.hpp"
 
 namespace tprh {
@@ -104,17 +109,6 @@ hipError_t launch_round_two_pass(const SplitArgs& p, size_t base, int cs, int m,
     return hipGetLastError();
 }
 
-// Workgroups of the one-pass kernel a device holds at once, with `lds`
-// bytes of LDS each (0 on a query error).
-template <typename K>
-int persistent_capacity(K kernel, size_t lds) {
-    int dev = 0, cus = 0, occ = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kPersistThreads, lds) != hipSuccess) return 0;
-    return cus * occ;
-}
-
 // Lag of the pipelined form in rows tasks: twice the workgroups resident at
 // once (capacity; its query failing gives 0), so that a task's waits are
 // normally over when it starts (measured on MI355X at 0.5, 1, 2 and 4 times
@@ -150,6 +144,21 @@ hipError_t launch_round_pipelined(const SplitArgs& p, size_t base, int cs, int m
     return hipGetLastError();
 }
 
+// The fast one-pass form (split_fused.hpp): s = 256 and more in fast PTPR.
+template <int METHOD, int MODE>
+constexpr bool kFusedSplit = METHOD == 0 && MODE == kFast;
+
+template <bool HAS_B, typename CT, bool REFINE>
+hipError_t launch_fused_rounds(const SplitArgs& p, int m, hipStream_t stream, bool* done) {
+    *done = true;
+    for (int s0 = 0; s0 < p.nsys && *done; s0 += p.chunk) {
+        const int cs = (p.nsys - s0 < p.chunk) ? p.nsys - s0 : p.chunk;
+        const hipError_t e = launch_fused<HAS_B, CT, REFINE>(round_loc<CT>(p, (size_t)s0 * p.n, m), p.n, cs, stream, done);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 template <int METHOD, int E, int L, int MODE, bool HAS_B, typename CT, bool REFINE>
 hipError_t launch_split_variant(const SplitArgs& p, int m, hipStream_t stream) {
     // a system is bps blocks of 256 lanes (m L > 1024 on this path, so bps
@@ -158,24 +167,29 @@ hipError_t launch_split_variant(const SplitArgs& p, int m, hipStream_t stream) {
     const int lg_bps = __builtin_ctz((unsigned)bps);
     const size_t lds = sizeof(float) * 10 * (size_t)m;
     const int lds_max = (int)(sizeof(float) * 10 * kSplitMaxM);
-    const auto pk = persistent_split_kernel<METHOD, E, L, MODE, HAS_B, CT, REFINE, BatchLoc<CT>>;
-    static std::atomic<unsigned long long> plds_set{0}, rlds_set{0};
-    hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(pk), lds_max, plds_set);
-    if (e == hipSuccess)
-        e = ensure_lds_limit(reinterpret_cast<const void*>(reduced_kernel<METHOD, BatchLoc<float>>), lds_max, rlds_set);
+    static std::atomic<unsigned long long> rlds_set{0};
+    hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(reduced_kernel<METHOD, BatchLoc<float>>), lds_max, rlds_set);
     if (e != hipSuccess) return e;
     // the one-pass form only when the caller asks for it (measured slower
     // than two passes on MI355X wherever a round has more blocks than the
     // chip holds at once: every wave of blocks waits out a reduced solve),
     // and only where every block of a system can be resident at once
-    const int capacity = p.form == 2 ? persistent_capacity(pk, lds) : 0;
+    int capacity = 0;
+    if constexpr (!(kFusedSplit<METHOD, MODE> && E >= 16)) {
+        if (p.form == 2) {
+            const auto pk = persistent_split_kernel<METHOD, E, L, MODE, HAS_B, CT, REFINE, BatchLoc<CT>>;
+            static std::atomic<unsigned long long> plds_set{0};
+            if ((e = ensure_lds_limit(reinterpret_cast<const void*>(pk), lds_max, plds_set)) != hipSuccess) return e;
+            capacity = resident_workgroups(pk, kPersistThreads, lds);
+        }
+    }
     const bool one_pass = p.form == 2 && capacity >= bps;
     int lag = 0, qcap = 0;
     if (p.form == 3) {
         const auto qk = pipelined_split_kernel<METHOD, E, L, MODE, HAS_B, CT, REFINE, BatchLoc<CT>>;
         static std::atomic<unsigned long long> qlds_set{0};
         if ((e = ensure_lds_limit(reinterpret_cast<const void*>(qk), lds_max, qlds_set)) != hipSuccess) return e;
-        qcap = persistent_capacity(qk, lds);
+        qcap = resident_workgroups(qk, kPersistThreads, lds);
         // the lag: about the workgroups the device holds at once, so that a
         // stage-3 task is normally taken after its system's reduced solve
         lag = pipeline_lag(qcap);
@@ -186,10 +200,11 @@ hipError_t launch_split_variant(const SplitArgs& p, int m, hipStream_t stream) {
         if (p.form == 3)
             e = launch_round_pipelined<METHOD, E, L, MODE, HAS_B, CT, REFINE>(p, base, cs, m, lg_bps, qcap, lag, lds,
                                                                               stream);
-        else if (one_pass)
-            e = launch_round_persistent<METHOD, E, L, MODE, HAS_B, CT, REFINE>(p, base, cs, m, lg_bps, capacity, lds,
-                                                                               stream);
-        else
+        else if (one_pass) {
+            if constexpr (!(kFusedSplit<METHOD, MODE> && E >= 16))
+                e = launch_round_persistent<METHOD, E, L, MODE, HAS_B, CT, REFINE>(p, base, cs, m, lg_bps, capacity,
+                                                                                   lds, stream);
+        } else
             e = launch_round_two_pass<METHOD, E, L, MODE, HAS_B, CT, REFINE>(p, base, cs, m, lds, stream);
         if (e != hipSuccess) return e;
     }
@@ -200,6 +215,23 @@ template <int METHOD, int E, int L, int MODE>
 hipError_t launch_split_el(const SplitArgs& p, hipStream_t stream) {
     const int m = p.n / (E * L);
     const bool hb = p.b != nullptr;
+    if constexpr (kFusedSplit<METHOD, MODE> && E >= 16) {
+        // the library's form, and the one-pass form, for s >= 256
+        if (p.form == 0 || p.form == 2) {
+            bool done = false;
+            hipError_t e;
+            if (p.f16)
+                e = hb ? launch_fused_rounds<true, _Float16, false>(p, m, stream, &done)
+                       : launch_fused_rounds<false, _Float16, false>(p, m, stream, &done);
+            else if (p.refine)
+                e = hb ? launch_fused_rounds<true, float, true>(p, m, stream, &done)
+                       : launch_fused_rounds<false, float, true>(p, m, stream, &done);
+            else
+                e = hb ? launch_fused_rounds<true, float, false>(p, m, stream, &done)
+                       : launch_fused_rounds<false, float, false>(p, m, stream, &done);
+            if (e != hipSuccess || done) return e;
+        }
+    }
     if (p.f16) {
         return hb ? launch_split_variant<METHOD, E, L, MODE, true, _Float16, false>(p, m, stream)
                   : launch_split_variant<METHOD, E, L, MODE, false, _Float16, false>(p, m, stream);

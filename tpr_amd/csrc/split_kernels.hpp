@@ -58,13 +58,12 @@ template <int METHOD, int E, int L, int MODE>
 constexpr bool kSplitTwoLevel = METHOD == 0 && MODE == kFast && L == 16 && E >= 2;
 
 // K1 and K3 load (and K3 stores) their slices as 1 KB runs per instruction
-// through LDS (staged_io.hpp) where the shape stages and the coefficients are
-// fp32: a wavefront holds 64 / L whole slices of one system (m L > 1024), one
+// through LDS (staged_io.hpp) where the shape stages: a wavefront holds 64 / L whole slices of one system (m L > 1024), one
 // contiguous run starting at `run`.  256-lane workgroups: four wavefronts.
 // K3 stores x non-temporally (256 x N=65536: 0.0951-0.0955 against
 // 0.0965-0.0968 ms with cached stores).
 template <int E, typename CT>
-constexpr bool kSplitStaged = kStageX<E> && std::is_same<CT, float>::value;
+constexpr bool kSplitStaged = kStageX<E>;
 template <int E, typename CT>
 constexpr int kSplitStageWords = kSplitStaged<E, CT> ? 4 * stage_wave_words<E>() : 4;
 
@@ -72,8 +71,8 @@ template <int E, bool HAS_B, typename CT, typename Loc>
 __device__ __forceinline__ void load_slices(const Loc& loc, long long q, size_t lo, size_t run, float* stage,
                                             RawPart<E>& raw) {
     if constexpr (kSplitStaged<E, CT>) {
-        load_raw_staged<E, HAS_B>(loc.A(q), HAS_B ? loc.B(q) : nullptr, loc.C(q), loc.D(q), run, (size_t)loc.n,
-                                  stage, threadIdx.x & 63, raw);
+        load_raw_staged<E, HAS_B, false, CT>(loc.A(q), HAS_B ? loc.B(q) : nullptr, loc.C(q), loc.D(q), run,
+                                             (size_t)loc.n, stage, threadIdx.x & 63, raw);
     } else {
         load_raw_t<E, CT>(loc.A(q), HAS_B ? loc.B(q) : nullptr, loc.C(q), loc.D(q), lo, lo, raw);
     }

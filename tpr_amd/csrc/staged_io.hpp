@@ -66,51 +66,90 @@ __device__ __forceinline__ void store_x_staged(float* __restrict__ x, const floa
     group_sync<true>();  // the area may be written again
 }
 
-// Loads the lane's E values of a, b (HAS_B), c and d from the wavefront's
-// run at `run`, as 1 KB per instruction.  Pieces at or past `total` load the
-// last piece before it instead (lanes that never store).  Every lane of the
-// wavefront calls this.
-template <int E, bool HAS_B>
-__device__ __forceinline__ void load_raw_staged(const float* __restrict__ a, const float* __restrict__ b,
-                                                const float* __restrict__ c, const float* __restrict__ d, size_t run,
-                                                size_t total, float* stage, int lane, RawPart<E>& p) {
-    constexpr int K = E / 4;
-    size_t gi[K];
+// The lane's E values of one array out of the 16-byte pieces that the
+// wavefront loaded of it (piece k * 64 + lane in l[k]), turned through LDS:
+// E / 4 pieces of floats, or E / 8 of fp16 values, widened (exact).
+template <int E>
+__device__ __forceinline__ void turn_run(const stage_v4f (&l)[E / 4], float* stage, int lane, float (&out)[E],
+                                         const float*) {
+    stage_v4f* s4 = reinterpret_cast<stage_v4f*>(stage);
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const size_t g = run + 4 * (size_t)(k * 64 + lane);
-        gi[k] = g < total ? g : total - 4;
+    for (int k = 0; k < E / 4; k++) s4[stage_slot(k * 64 + lane)] = l[k];
+    group_sync<true>();
+#pragma unroll
+    for (int i = 0; i < E / 4; i++) {
+        const stage_v4f v = s4[stage_slot(lane * (E / 4) + i)];
+        out[4 * i] = v.x;
+        out[4 * i + 1] = v.y;
+        out[4 * i + 2] = v.z;
+        out[4 * i + 3] = v.w;
     }
-    stage_v4f la[K], lb[K], lc[K], ld[K];
+    group_sync<true>();
+}
+template <int E>
+__device__ __forceinline__ void turn_run(const stage_v4f (&l)[E / 8], float* stage, int lane, float (&out)[E],
+                                         const _Float16*) {
+    typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+    stage_v4f* s4 = reinterpret_cast<stage_v4f*>(stage);
+    if constexpr (E > 8) {
 #pragma unroll
-    for (int k = 0; k < K; k++) la[k] = *reinterpret_cast<const stage_v4f*>(a + gi[k]);
+        for (int k = 0; k < E / 8; k++) s4[stage_slot(k * 64 + lane)] = l[k];
+        group_sync<true>();
+    }
 #pragma unroll
-    for (int k = 0; k < K; k++) lc[k] = *reinterpret_cast<const stage_v4f*>(c + gi[k]);
+    for (int i = 0; i < E / 8; i++) {
+        const stage_v4f w = E > 8 ? s4[stage_slot(lane * (E / 8) + i)] : l[0];
+        const v8h v = __builtin_bit_cast(v8h, w);
 #pragma unroll
-    for (int k = 0; k < K; k++) ld[k] = *reinterpret_cast<const stage_v4f*>(d + gi[k]);
+        for (int k = 0; k < 8; k++) out[8 * i + k] = (float)v[k];
+    }
+    if constexpr (E > 8) group_sync<true>();
+}
+
+// Loads the lane's E values of a, b (HAS_B), c (float or fp16) and d from the
+// wavefront's run at `run`, as 1 KB per instruction.  CLAMP: pieces at or
+// past `total` load the last piece before it instead (lanes that never
+// store); without it the whole run lies below `total`.  Every lane of the
+// wavefront calls this.
+template <int E, bool HAS_B, bool CLAMP = true, typename CT = float>
+__device__ __forceinline__ void load_raw_staged(const CT* __restrict__ a, const CT* __restrict__ b,
+                                                const CT* __restrict__ c, const float* __restrict__ d, size_t run,
+                                                size_t total, float* stage, int lane, RawPart<E>& p) {
+    constexpr int V = 16 / (int)sizeof(CT);  // values per piece
+    constexpr int K = E / V;                 // pieces per lane
+    // the lane's k-th piece of an array of v values per piece
+    auto load = [&](const auto* q, int k, int v) {
+        size_t g = run + (size_t)v * (size_t)(k * 64 + lane);
+        if (CLAMP) g = g < total ? g : total - (size_t)v;
+        return *reinterpret_cast<const stage_v4f*>(q + g);
+    };
+    stage_v4f la[K], lb[K], lc[K], ld[E / 4];
+#pragma unroll
+    for (int k = 0; k < K; k++) la[k] = load(a, k, V);
+#pragma unroll
+    for (int k = 0; k < K; k++) lc[k] = load(c, k, V);
+#pragma unroll
+    for (int k = 0; k < E / 4; k++) ld[k] = load(d, k, 4);
     if constexpr (HAS_B) {
 #pragma unroll
-        for (int k = 0; k < K; k++) lb[k] = *reinterpret_cast<const stage_v4f*>(b + gi[k]);
+        for (int k = 0; k < K; k++) lb[k] = load(b, k, V);
     }
-    stage_v4f* s4 = reinterpret_cast<stage_v4f*>(stage);
-    auto turn = [&](const stage_v4f(&l)[K], float(&out)[E]) {
-#pragma unroll
-        for (int k = 0; k < K; k++) s4[stage_slot(k * 64 + lane)] = l[k];
-        group_sync<true>();
-#pragma unroll
-        for (int i = 0; i < K; i++) {
-            const stage_v4f v = s4[stage_slot(lane * K + i)];
-            out[4 * i] = v.x;
-            out[4 * i + 1] = v.y;
-            out[4 * i + 2] = v.z;
-            out[4 * i + 3] = v.w;
-        }
-        group_sync<true>();
-    };
-    turn(la, p.a);
-    turn(lc, p.c);
-    turn(ld, p.d);
-    if constexpr (HAS_B) turn(lb, p.b);
+    turn_run<E>(la, stage, lane, p.a, a);
+    turn_run<E>(lc, stage, lane, p.c, a);
+    turn_run<E>(ld, stage, lane, p.d, d);
+    if constexpr (HAS_B) turn_run<E>(lb, stage, lane, p.b, a);
+}
+
+// x just before and just after the lane's E values xo: from the lanes beside
+// it, at the wavefront's ends from memory (0 outside the system's [0, n)).
+// lo: the lane's first equation in the system at x.
+template <int E>
+__device__ __forceinline__ void wave_halo(const float* __restrict__ x, size_t lo, int n, int lane,
+                                          const float (&xo)[E], float& xl, float& xr) {
+    xl = shift_up<64, 1>(xo[E - 1], 0.0f, lane);
+    xr = shift_down<64, 1>(xo[0], 0.0f, lane);
+    if (lane == 0 && lo > 0) xl = x[lo - 1];
+    if (lane == 63 && lo + E < (size_t)n) xr = x[lo + E];
 }
 
 }  // namespace tprh

@@ -14,7 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../csrc/slice_solvers.hpp"
-#include "../csrc/split_kernels.hpp"
+#include "../csrc/split_fused.hpp"
 #include "../csrc/staged_io.hpp"
 
 namespace tprh {
@@ -150,6 +150,42 @@ extern "C" int tprh_diag_ptpr_stage_clock(const float* a, const float* b, const 
         case 8: hipLaunchKernelGGL(ptpr_stage_clock_kernel<8>, dim3(grid), dim3(kClockBlock), shmem, st, a, b, c, d, x, n, m, nsys, lg, stamps); break;
         default: hipLaunchKernelGGL(ptpr_stage_clock_kernel<16>, dim3(grid), dim3(kClockBlock), shmem, st, a, b, c, d, x, n, m, nsys, lg, stamps); break;
     }
+    return (int)hipGetLastError();
+}
+
+// The one-pass split solve (split_fused.hpp) of nsys fast-PTPR systems of n
+// equations with a diagonal, fp32, run by `blocks` workgroups as the
+// first .. first + blocks - 1 of `stride`, each giving up a wait after `spin`
+// polls: a sweep whose workgroups are not all there, which lists its tiles
+// and publishes the absent ones'.  clear: empty the published words first
+// (the first of several launches that make up one solve).  workspace as
+// tprh_workspace_bytes gives for s = 256, chunk = nsys.  Returns a hipError_t.
+extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float* c, const float* d, float* x, int n,
+                                     int nsys, int refine, void* workspace, int clear, int first, int blocks,
+                                     int stride, int spin, void* stream) {
+    using namespace tprh;
+    const int m = n / 256;
+    if (n % kFusedTile || (n & (n - 1)) || m > kSplitMaxM || nsys < 1 || first < 0 || blocks < 1 ||
+        first + blocks > stride || spin < 0)
+        return (int)hipErrorInvalidValue;
+    SplitArgs p{};
+    split_carve(workspace, m, nsys, &p);
+    BatchLoc<float> loc;
+    loc.a = a, loc.b = b, loc.c = c, loc.d = d, loc.x = x;
+    loc.rows = p.rows, loc.xed = p.xed, loc.n = n, loc.m = m, loc.cstride = (size_t)n;
+    const int lg = __builtin_ctz((unsigned)(n / kFusedTile));
+    hipStream_t st = (hipStream_t)stream;
+    if (clear) {
+        const int tiles = nsys << lg;
+        hipLaunchKernelGGL((clear_fused_kernel<BatchLoc<float>>), dim3((tiles + 255) / 256), dim3(256), 0, st, loc, nsys,
+                           lg);
+    }
+    const bool wide = (1 << lg) > kFusedWave;
+    auto* kern = refine ? (wide ? fused_split_kernel<true, float, true, true, BatchLoc<float>>
+                                : fused_split_kernel<true, float, true, false, BatchLoc<float>>)
+                        : (wide ? fused_split_kernel<true, float, false, true, BatchLoc<float>>
+                                : fused_split_kernel<true, float, false, false, BatchLoc<float>>);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), 0, st, loc, nsys, lg, first, stride, spin);
     return (int)hipGetLastError();
 }
 
