@@ -178,12 +178,12 @@ typedef struct tprh_solve_desc {
     int coef_shared;        /* 1: every system uses the one matrix at a, b, c (n values each):
                                nsys right-hand sides of one matrix, as in ADI sweeps */
     int split_form;         /* systems above one workgroup: 0 = chosen by the library (one pass
-                               for fast PTPR with s >= 256, else two passes); 1 = two passes
+                               in fast arithmetic with s >= 256, else two passes); 1 = two passes
                                (stage 1 and the reduced systems, then stage 3, which reads the
                                inputs again: 36 B/eq); 2 = one pass (each slice stays in
                                registers from load to store, 20 B/eq, where every workgroup of a
-                               system can be resident at once, else two passes; outside fast PTPR
-                               with s >= 256 slower than two passes when a round has more
+                               system can be resident at once, else two passes; in exact arithmetic or
+                               with s < 256 slower than two passes when a round has more
                                workgroups than the device holds); 3 = pipelined (one persistent launch of
                                rows, reduced-system and stage-3 tasks; slower than two passes
                                on MI355X).  Exact answers are the same bits in every form. */
@@ -192,7 +192,7 @@ typedef struct tprh_solve_desc {
                                for launches overlapping on several streams); 1 = x written
                                through the caches, for a caller whose next kernel reads x.
                                Same answers either way.  Larger systems: two passes, and one
-                               pass in fast PTPR with s >= 256, write x non-temporally, the
+                               pass in fast arithmetic with s >= 256, write x non-temporally, the
                                others through the caches, whatever this flag says. */
 } tprh_solve_desc;
 

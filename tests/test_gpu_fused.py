@@ -1,4 +1,4 @@
-"""The one-pass form of fast PTPR on systems larger than one workgroup
+"""The one-pass form of fast PTPR and TPR on systems larger than one workgroup
 (split_fused.hpp): tiles of 4096 equations that exchange six numbers each.
 
 Sizes at its edges: 8, 16 (one DPP row of tiles), 32 and 64 (several rows in
@@ -45,11 +45,12 @@ def bits(t):
 
 @pytest.mark.parametrize("n,s,nsys", [(32768, 256, 3), (65536, 256, 5), (65536, 2048, 3), (131072, 512, 3),
                                       (262144, 256, 2), (524288, 1024, 3), (1 << 22, 2048, 1)])
-def test_one_pass_forms_agree(n, s, nsys):
+@pytest.mark.parametrize("method", ["ptpr", "tpr"])
+def test_one_pass_forms_agree(method, n, s, nsys):
     """Diagonal, unit diagonal, fp16 storage, a shared matrix, a refinement
     step: the one-pass form against the two passes and the oracle, and
     nothing written past x."""
-    say("one pass", n, s, nsys)
+    say("one pass", method, n, s, nsys)
     a, b, c, d, _ = O.gen_batch(61, 0, nsys, n)
     da, db, dc, dd = dev(a), dev(b), dev(c), dev(d)
     guard = 4096
@@ -59,13 +60,13 @@ def test_one_pass_forms_agree(n, s, nsys):
         x = torch.full((nsys * n + guard,), 2.5, device="cuda")
         if x0 is not None:
             x[:nsys * n] = x0
-        B.solve_ex(*coef, dd, x[:nsys * n], n, s, split_form=form, **kw)
+        B.solve_ex(*coef, dd, x[:nsys * n], n, s, split_form=form, method=method, **kw)
         torch.cuda.synchronize()
         assert bool((x[nsys * n:] == 2.5).all())
         return x[:nsys * n].clone()
 
     x = solve(0, (da, db, dc))
-    assert rel(x.cpu().numpy(), O.solve_batch("ptpr", a, b, c, d, n, s), n) <= FAST_TOL
+    assert rel(x.cpu().numpy(), O.solve_batch(method, a, b, c, d, n, s), n) <= FAST_TOL
     assert np.array_equal(bits(x), bits(solve(2, (da, db, dc))))
     cases = [((da, db, dc), {}), ((da / db, None, dc / db), {}), ([v.half() for v in (da, db, dc)], {}),
              ([v[:n].contiguous() for v in (da, db, dc)], {"shared": True}),
@@ -76,9 +77,10 @@ def test_one_pass_forms_agree(n, s, nsys):
 
 
 @pytest.mark.parametrize("n,s,nsys", [(65536, 256, 70), (524288, 512, 9)])
-def test_one_pass_weakly_dominant_accuracy(n, s, nsys):
+@pytest.mark.parametrize("method", ["ptpr", "tpr"])
+def test_one_pass_weakly_dominant_accuracy(method, n, s, nsys):
     """More tiles than the device holds at once, weakly dominant."""
-    say("one pass, weak", n, s, nsys)
+    say("one pass, weak", method, n, s, nsys)
     t = B.alloc_batch(nsys, n)
     B.generate("weak", 62, 0, nsys, n, t["a"], t["b"], t["c"], t["d"], t["xt"])
     a, b, c, d = (t[k].cpu().numpy() for k in "abcd")
@@ -86,7 +88,7 @@ def test_one_pass_weakly_dominant_accuracy(n, s, nsys):
     err = {}
     for form in (0, 1):
         for refine in (False, True):
-            B.solve_ex(t["a"], t["b"], t["c"], t["d"], t["x"], n, s, split_form=form, refine=refine)
+            B.solve_ex(t["a"], t["b"], t["c"], t["d"], t["x"], n, s, split_form=form, refine=refine, method=method)
             torch.cuda.synchronize()
             err[form, refine] = rel(t["x"].cpu().numpy(), ref, n)
     say(err)

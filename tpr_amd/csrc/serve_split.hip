@@ -29,11 +29,11 @@ namespace {
 template <int METHOD, int E, int L, int MODE>
 hipError_t launch_el(const ServeSplitLaunch& p, hipStream_t stream) {
     const int m = p.n / (E * L);
-    if constexpr (METHOD == 0 && MODE == kFast) {
+    if constexpr (MODE == kFast) {
         // one pass (split_fused.hpp); every shape here has s >= 256
         bool done = false;
         const hipError_t e =
-            launch_fused<true, float, false>(TableLoc{p.sys, p.base, p.n, m}, p.n, p.nsys, stream, &done);
+            launch_fused<METHOD, true, float, false>(TableLoc{p.sys, p.base, p.n, m}, p.n, p.nsys, stream, &done);
         if (e != hipSuccess || done) return e;
     }
     const int lg_m = __builtin_ctz((unsigned)m);

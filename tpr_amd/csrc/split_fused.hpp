@@ -1,13 +1,13 @@
-// split_fused.hpp -- fast PTPR on systems larger than one workgroup in one
-// pass: every equation is read once and x written once (20 B/eq), against 36
-// B/eq for the two passes of split_kernels.hpp.
+// split_fused.hpp -- fast PTPR and TPR on systems larger than one workgroup in
+// one pass: every equation is read once and x written once (20 B/eq), against
+// 36 B/eq for the two passes of split_kernels.hpp.
 //
 // What bounds it: HBM.  The two passes move 604 MB for 256 x N=65536 at the
 // rate such bytes can be moved (K1 46, K2 6, K3 47 us); reading the inputs
-// once leaves 336 MB.  A whole solve of that batch: 101 us two passes, 65 us
-// this way (5.1 TB/s; a device copy of that size reaches 4.8-5.4); with an
-// fp16-stored solve and a refinement step 203 -> 134 us; one system of 1 Mi
-// equations 29 -> 21 us.
+// once leaves 336 MB.  A whole solve of that batch: 101 us two passes, 63.5
+// us this way (5.3 TB/s; a device copy of that size reaches 4.8-5.4); with an
+// fp16-stored solve and a refinement step 203 -> 129 us; one system of 1 Mi
+// equations 29 -> 14 us.
 //
 // A tile is 4096 consecutive equations of one system: 256 lanes x 16, sixteen
 // rows of 16 lanes (one DPP row, 256 equations).  A workgroup
@@ -21,8 +21,8 @@
 //      for another;
 //   3. publishes those six numbers, and waits for the other tiles' of its
 //      system with its equations' state still in registers;
-//   4. solves the system of the tiles' last unknowns by the same steps (one
-//      tile per lane) and finishes its rows from the unknowns on either side
+//   4. solves the system of the tiles' ends by the same steps (one tile per
+//      lane) and finishes its rows from the unknowns on either side
 //      of the tile (src/ptpr.cpp:263-287, x[ed+1] from the next row's first
 //      equation instead of a division by c_ed).
 // So one exchange of 24 bytes per 4096 equations crosses the chip, and the
@@ -30,12 +30,14 @@
 // counter: the words are device-coherent, set to a NaN pattern that is never
 // published before the launch (clear_fused_kernel), and a reader polls until
 // no word of that pattern is left.  Four workgroups live on a CU at once, so
-// that one's wait (4.3 us of a tile's 12 at the median) is covered by others'
+// that one's wait (4.1 us of a tile's 11 at the median) is covered by others'
 // loads.
 //
 // Slices: s = 256 (one row), 512, 1024 or 2048 (several rows) -- in fast
 // arithmetic a slice's interior, and the rows of a tile, may be eliminated in
-// any order.
+// any order.  TPR runs its tree stages on every row instead of the two-level
+// form, everything else alike (256 x N=65536, one
+// buffer set: 100 us two passes, 58 us).
 //
 // The solve ends whichever workgroups are resident.  Workgroup k of a grid of
 // G takes tiles k, k + G, ...; it publishes a tile before it waits, and waits
@@ -59,7 +61,6 @@ namespace tprh {
 constexpr int kFusedTile = 4096;               // equations per workgroup
 constexpr int kFusedThreads = 256;
 constexpr int kFusedGroup = 16;                // tiles per group (one DPP row)
-constexpr int kFusedWave = 64;                 // blocks of a chain that one wavefront solves
 constexpr unsigned kFusedEmpty = 0xffffffffu;  // a word not yet published
 constexpr int kFusedSpin = 64;                 // polls (about a microsecond each) before a tile is listed
 constexpr int kFusedTries = 1 << 14;           // tasks of one workgroup beyond its own tiles, in all
@@ -68,35 +69,45 @@ constexpr int kFusedTries = 1 << 14;           // tasks of one workgroup beyond 
 // or one of another workgroup published on its behalf.
 enum FusedKind { kFusedOwn = 0, kFusedAgain = 1, kFusedHelp = 2 };
 
-// A system's boundary buffer (Rows) of bps tiles holds: words 8 t .. 8 t + 7
-// what tile t publishes, its equations [F.a, F.c, F.r, L.a, L.c, L.r] (F:
-// first unknown, L: last) and, with refinement, the iterate's x at both; from
-// 8 bps one word per tile, the list link; from 9 bps eight words per group of
-// 16 tiles, its equations.  9.5 words per tile in all; the buffer has 8 per
-// slice, two slices or more per tile.
-__device__ __forceinline__ int* fused_link(float* rows, int bps, int t) {
-    return reinterpret_cast<int*>(rows) + 8 * (size_t)bps + t;
-}
-__device__ __forceinline__ float* fused_groups(float* rows, int bps) { return rows + 9 * (size_t)bps; }
-
-// Marks every published word empty: one thread per tile (a kernel, not a
-// memset, so that a captured graph replays it).
-template <typename Loc>
-__global__ __launch_bounds__(256) void clear_fused_kernel(Loc loc, int nsys, int lg_bps) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nsys << lg_bps) return;
-    const int bps = 1 << lg_bps;
-    const int t = i & (bps - 1);
-    float* rows = loc.Rows(i >> lg_bps);
-    const uint4 e = make_uint4(kFusedEmpty, kFusedEmpty, kFusedEmpty, kFusedEmpty);
-    uint4* w = reinterpret_cast<uint4*>(rows + 8 * (size_t)t);
-    w[0] = e;
-    w[1] = e;
-    if (bps > kFusedWave && t % kFusedGroup == 0) {
-        w = reinterpret_cast<uint4*>(fused_groups(rows, bps) + 8 * (t / kFusedGroup));
-        w[0] = e;
-        w[1] = e;
+// What the workgroups of one system exchange, in its boundary buffer (Rows)
+// of bps tiles.  For block t (a tile; behind them a group of 16 tiles), its
+// equations [F.a, F.c, F.r, L.a, L.c, L.r] (F: first unknown, L: last) are
+// four words at ends4(t) and two at ends2(t), so that a wavefront reads 16
+// blocks' words as three 128-byte lines: reads of one line from all over the
+// chip are served one after the other, and polls are most of them.  x2: the
+// iterate's x at a tile's ends (refinement); result: x just before and after
+// a tile, found by its group's first; link: the list.  11 3/8 words per tile
+// in all; the buffer has 8 per slice, two slices or more per tile.
+struct FusedWords {
+    float* rows;
+    int bps;
+    __device__ __forceinline__ int groups() const { return bps / kFusedGroup; }
+    __device__ __forceinline__ float* ends4(int t) const { return rows + 4 * (size_t)t; }
+    __device__ __forceinline__ float* ends2(int t) const { return rows + 4 * (size_t)bps + 2 * (size_t)t; }
+    __device__ __forceinline__ float* x2(int t) const { return rows + 6 * (size_t)bps + 2 * (size_t)t; }
+    __device__ __forceinline__ float* result(int t) const { return rows + 8 * (size_t)bps + 2 * (size_t)t; }
+    __device__ __forceinline__ int* link(int t) const { return reinterpret_cast<int*>(rows) + 10 * (size_t)bps + t; }
+    __device__ __forceinline__ float* group4(int g) const { return rows + 11 * (size_t)bps + 4 * g; }
+    __device__ __forceinline__ float* group2(int g) const {
+        return rows + 11 * (size_t)bps + 4 * (size_t)groups() + 2 * g;
     }
+};
+
+// Marks every published word empty (a kernel, not a memset, so that a
+// captured graph replays it): the 10 words per tile ahead of the list links
+// and the groups' behind them, in 16-byte pieces, one per thread.
+__host__ __device__ inline int fused_clear_pieces(int bps) {
+    return (10 * bps + (bps > kFusedGroup ? 6 * (bps / kFusedGroup) : 0)) / 4;
+}
+template <typename Loc>
+__global__ __launch_bounds__(256) void clear_fused_kernel(Loc loc, int nsys, int bps) {
+    const int pieces = fused_clear_pieces(bps);
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (long long)nsys * pieces) return;
+    const int q = (int)(i / pieces);
+    int k = (int)(i - (long long)q * pieces);
+    if (4 * k >= 10 * bps) k += bps / 4;  // the list links are not cleared
+    reinterpret_cast<uint4*>(loc.Rows(q))[k] = make_uint4(kFusedEmpty, kFusedEmpty, kFusedEmpty, kFusedEmpty);
 }
 
 // Equations of the first and last unknown of a block (a row, a tile, a group)
@@ -127,28 +138,58 @@ __device__ __forceinline__ float pair_second(unsigned long long v) {
     return __builtin_bit_cast(float, (unsigned)(v >> 32));
 }
 
-__device__ __forceinline__ void publish_ends(float* p, const BlockEnds& e) {
-    publish_pair(p, e.fa, e.fc);
-    publish_pair(p + 2, e.fr, e.la);
-    publish_pair(p + 4, e.lc, e.lr);
+__device__ __forceinline__ void publish_ends(float* p4, float* p2, const BlockEnds& e) {
+    publish_pair(p4, e.fa, e.fc);
+    publish_pair(p4 + 2, e.fr, e.la);
+    publish_pair(p2, e.lc, e.lr);
 }
-// False while a word is missing.
-__device__ __forceinline__ bool read_ends(const float* p, BlockEnds& e) {
-    const unsigned long long v0 = read_pair(p), v1 = read_pair(p + 2), v2 = read_pair(p + 4);
-    e = BlockEnds{pair_first(v0), pair_second(v0), pair_first(v1), pair_second(v1), pair_first(v2), pair_second(v2)};
-    return !pair_missing(v0) && !pair_missing(v1) && !pair_missing(v2);
+// False while a word is missing.  Two device-coherent loads (every word is
+// checked by itself, so nothing wider than a word need be atomic).
+__device__ __forceinline__ bool read_ends(const float* p4, const float* p2, BlockEnds& e) {
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    v4u a;
+    v2u b;
+    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\t"
+                 "global_load_dwordx2 %1, %3, off sc1\n\t"
+                 "s_waitcnt vmcnt(0)"
+                 : "=&v"(a), "=&v"(b)
+                 : "v"(p4), "v"(p2)
+                 : "memory");
+    auto f = [](unsigned v) { return __builtin_bit_cast(float, v); };
+    e = BlockEnds{f(a.x), f(a.y), f(a.z), f(a.w), f(b.x), f(b.y)};
+    return a.x != kFusedEmpty && a.y != kFusedEmpty && a.z != kFusedEmpty && a.w != kFusedEmpty &&
+           b.x != kFusedEmpty && b.y != kFusedEmpty;
 }
 
-// Polls until lanes with `need` have read their blocks' words at p into
-// their e; after `limit` polls gives up.  Returns the lanes still missing
-// theirs.  Every lane of the wavefront calls this.
-__device__ __forceinline__ unsigned long long wait_ends(const float* p, bool need, int limit, BlockEnds& e) {
+// Polls until lanes with `need` have read their blocks' words into their e;
+// after `limit` polls gives up.  Returns the lanes still missing theirs.
+// Every lane of the wavefront calls this.
+__device__ __forceinline__ unsigned long long wait_ends(const float* p4, const float* p2, bool need, int limit,
+                                                        BlockEnds& e) {
     for (int i = 0;; i++) {
-        if (need) need = !read_ends(p, e);
+        if (need) need = !read_ends(p4, p2, e);
         const unsigned long long missing = __ballot(need);
         if (missing == 0 || i >= limit) return missing;
-        __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_s_sleep(2);
     }
+}
+// The same for one published pair, in lane 0.
+__device__ __forceinline__ unsigned long long wait_pair(const float* p, int lane, int limit, float& x, float& y) {
+    unsigned long long v = 0, missing;
+    bool need = lane == 0;
+    for (int i = 0;; i++) {
+        if (need) {
+            v = read_pair(p);
+            need = pair_missing(v);
+        }
+        missing = __ballot(need);
+        if (missing == 0 || i >= limit) break;
+        __builtin_amdgcn_s_sleep(2);
+    }
+    x = pair_first(v);
+    y = pair_second(v);
+    return missing;
 }
 
 // A chain of 16 blocks, one per lane of a DPP row, reduced to the unknowns
@@ -197,15 +238,17 @@ struct Chain16 {
     }
 };
 
-// A whole system of up to 64 blocks, one per lane (lanes past the last one
-// hold zero equations): x just before and just after block k (uniform).
+// A whole system of up to 16 blocks, with ROWS up to 64, one per lane (lanes
+// past the last one hold zero equations): x just before and just after block
+// k (uniform).
+template <bool ROWS>
 __device__ __forceinline__ void solve_blocks(const BlockEnds& e, int count, int k, int lane, float& before,
                                              float& after) {
     const int l = lane & 15;
     Chain16 c;
     c.reduce(e, l);
     float ob = 0.0f, oa = 0.0f;  // x outside the lane's row
-    if (count > 16) {
+    if (ROWS && count > 16) {
         // the (at most four) rows' ends, row r in lane r of every row
         BlockEnds u = c.ends(lane & 48);
         auto gather = [&](float v) {
@@ -227,10 +270,50 @@ __device__ __forceinline__ void solve_blocks(const BlockEnds& e, int count, int 
     after = k + 1 < count ? __shfl(xa, k, 64) : 0.0f;
 }
 
-// WIDE: more than kFusedWave tiles per system (up to 1024): the exchange is
-// in two steps, the tiles of a group of 16 first, the groups then, so that a
-// tile reads 16 + bps / 16 blocks' words instead of bps.
-template <bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
+// One lane's equations between the two halves of a row's solve: stage 1 into
+// the row's ends (sA, sC, sR in lane 0; eA, eC, eR in lane 15), and x from
+// the unknowns around the row once they are known.
+template <int METHOD, int E>
+struct RowState;
+template <int E>
+struct RowState<0, E> {  // PTPR: the two-level stage 1
+    Fast16State<E> st;
+    __device__ __forceinline__ void reduce(const RawPart<E>& raw, bool has_b, int l, BlockEnds& e) {
+        fast16_stage1<E>(raw, has_b, l, st);
+        e = BlockEnds{st.sA, st.sC, st.sR, st.eA, st.eC, st.eR};
+    }
+    __device__ __forceinline__ void finish(float before, float last, float after, int l, float (&X)[E]) const {
+        fast16_finish<E>(st, before, last, after, l, X);
+    }
+};
+template <int E>
+struct RowState<1, E> {  // TPR: the tree (src/tpr.cpp:123-230, :277-308)
+    float A[E], C[E], R[E], Ao[E], Co[E], Ro[E];
+    __device__ __forceinline__ void reduce(const RawPart<E>& raw, bool has_b, int l, BlockEnds& e) {
+        normalise<E, kFast>(raw, has_b, A, C, R);
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            Ao[i] = A[i];
+            Co[i] = C[i];
+            Ro[i] = R[i];
+        }
+        tpr_stage1_level<E, 16, kFast, 1>(A, C, R, l);
+        e = BlockEnds{A[0], C[0], R[0], A[E - 1], C[E - 1], R[E - 1]};
+    }
+    __device__ __forceinline__ void finish(float before, float last, float, int l, float (&X)[E]) const {
+        tpr_stage3<E, 16, kFast>(A, C, R, Ao, Co, Ro, before, last, l, X);
+    }
+};
+
+// WIDE: more than 16 tiles per system (up to 1024): the exchange goes through
+// groups of 16 tiles -- the group's first tile reduces it, exchanges its ends
+// with the other groups', and hands every tile of the group the x on its
+// sides -- so that a tile polls one word pair and no line is polled by more
+// than 64 workgroups.  Reads of one line from all over the chip are served
+// one after the other: with every tile polling every group's words, 16
+// systems of 1 Mi equations took 237 us, this way 78; with every tile polling
+// all of up to 64 tiles' words, 64 systems of 256 Ki 73 us, this way 59.
+template <int METHOD, bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
 __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_kernel(Loc loc, int nsys, int lg_bps, int first,
                                                                                     int stride, int spin) {
     constexpr int E = 16;
@@ -257,8 +340,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
     while (tile >= 0 && tile < total) {  // uniform
         const int q = tile >> lg_bps;
         const int ti = tile & (bps - 1);
-        float* rows = loc.Rows(q);
-        float* words = rows + 8 * (size_t)ti;
+        const FusedWords fw{loc.Rows(q), bps};
         const size_t lo = (size_t)ti * kFusedTile + (size_t)threadIdx.x * E;
         const size_t run = lo - (size_t)lane * E;
         RawPart<E> raw;
@@ -275,30 +357,31 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             float xl, xr;
             wave_halo<E>(loc.X(q), lo, loc.n, lane, xo, xl, xr);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads are complete before the reads below
-            if (lane == 0) seen = read_pair(words);
+            if (lane == 0) seen = read_pair(fw.ends2(ti));
             if (kind != kFusedOwn) {
                 if (threadIdx.x == 0 && ti > 0) {
-                    const unsigned long long v = read_pair(words - 2);
+                    const unsigned long long v = read_pair(fw.x2(ti - 1));
                     if (!pair_missing(v)) xl = pair_second(v);
                 }
                 if (threadIdx.x == kFusedThreads - 1 && ti + 1 < bps) {
-                    const unsigned long long v = read_pair(words + 14);
+                    const unsigned long long v = read_pair(fw.x2(ti + 1));
                     if (!pair_missing(v)) xr = pair_first(v);
                 }
             }
             residual_fp64<E, HAS_B>(xo, xl, xr, raw);
         }
-        Fast16State<E> fs;
-        fast16_stage1<E>(raw, HAS_B, l, fs);
+        RowState<METHOD, E> row;
+        BlockEnds re;
+        row.reduce(raw, HAS_B, l, re);
         if (l == 0) {
-            s_ends[0][j] = fs.sA;
-            s_ends[1][j] = fs.sC;
-            s_ends[2][j] = fs.sR;
+            s_ends[0][j] = re.fa;
+            s_ends[1][j] = re.fc;
+            s_ends[2][j] = re.fr;
         }
         if (l == 15) {
-            s_ends[3][j] = fs.eA;
-            s_ends[4][j] = fs.eC;
-            s_ends[5][j] = fs.eR;
+            s_ends[3][j] = re.la;
+            s_ends[4][j] = re.lc;
+            s_ends[5][j] = re.lr;
         }
         if constexpr (REFINE) {
             if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(seen) ? 0 : 1;
@@ -322,39 +405,46 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             const bool skip = REFINE && kind == kFusedHelp && (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
             const BlockEnds mine = ch.ends(0);
             if (threadIdx.x == 0 && kind != kFusedAgain && !skip) {
-                if constexpr (REFINE) publish_pair(words + 6, xo[0], s_xlast);
-                publish_ends(words, mine);
+                if constexpr (REFINE) publish_pair(fw.x2(ti), xo[0], s_xlast);
+                publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
             }
             BlockEnds e{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             float before = 0.0f, after = 0.0f;
             unsigned long long m;  // lanes whose block is missing
             const int limit = kind == kFusedHelp ? 0 : spin;
             if constexpr (!WIDE) {
-                m = wait_ends(rows + 8 * (size_t)lane, lane < bps, limit, e);
-                if (m == 0) solve_blocks(e, bps, ti, lane, before, after);
+                m = wait_ends(fw.ends4(lane), fw.ends2(lane), lane < bps, limit, e);
+                if (m == 0) solve_blocks<false>(e, bps, ti, lane, before, after);
                 else missing = tile - ti + __builtin_ctzll(m);
             } else {
-                const int g = ti / kFusedGroup, ng = bps / kFusedGroup;
-                m = wait_ends(rows + 8 * (size_t)(g * kFusedGroup + l), lane < kFusedGroup, limit, e);
-                if (m != 0) {
-                    missing = tile - ti + g * kFusedGroup + __builtin_ctzll(m);
+                const int g = ti / kFusedGroup, ng = fw.groups();
+                // the group's first tile reduces the group, solves the system
+                // of the groups and hands every tile of the group its sides
+                // (a tile taken up again does so by itself)
+                if (ti % kFusedGroup != 0 && kind == kFusedOwn) {
+                    m = wait_pair(fw.result(ti), lane, limit, before, after);
                 } else {
-                    Chain16 cg;
-                    cg.reduce(e, l);
-                    // every tile of the group publishes its equations (the
-                    // same words), so that none waits for a particular one
-                    const BlockEnds ge = cg.ends(0);
-                    if (threadIdx.x == 0) publish_ends(fused_groups(rows, bps) + 8 * g, ge);
-                    e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-                    m = wait_ends(fused_groups(rows, bps) + 8 * lane, lane < ng, limit, e);
+                    const int t = g * kFusedGroup + l;
+                    m = wait_ends(fw.ends4(t), fw.ends2(t), lane < kFusedGroup, limit, e);
                     if (m != 0) {
-                        missing = tile - ti + __builtin_ctzll(m) * kFusedGroup + tries % kFusedGroup;
+                        missing = tile - ti + g * kFusedGroup + __builtin_ctzll(m);
                     } else {
-                        float ob, oa, xb, xe, xa;
-                        solve_blocks(e, ng, g, lane, ob, oa);
-                        cg.solve(ob, oa, l, xb, xe, xa);
-                        before = __shfl(xb, ti % kFusedGroup, 64);
-                        after = __shfl(xa, ti % kFusedGroup, 64);
+                        Chain16 cg;
+                        cg.reduce(e, l);
+                        const BlockEnds ge = cg.ends(0);
+                        if (threadIdx.x == 0) publish_ends(fw.group4(g), fw.group2(g), ge);
+                        e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+                        m = wait_ends(fw.group4(lane), fw.group2(lane), lane < ng, limit, e);
+                        if (m != 0) {
+                            missing = tile - ti + __builtin_ctzll(m) * kFusedGroup + tries % kFusedGroup;
+                        } else {
+                            float ob, oa, xb, xe, xa;
+                            solve_blocks<true>(e, ng, g, lane, ob, oa);
+                            cg.solve(ob, oa, l, xb, xe, xa);
+                            if (lane < kFusedGroup) publish_pair(fw.result(t), xb, xa);
+                            before = __shfl(xb, ti % kFusedGroup, 64);
+                            after = __shfl(xa, ti % kFusedGroup, 64);
+                        }
                     }
                 }
             }
@@ -371,7 +461,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             ch.solve(s_side[0], s_side[1], l, xb, xe, xa);
             const int src = (lane & 48) + j;  // a lane that holds row j
             float X[E];
-            fast16_finish<E>(fs, __shfl(xb, src, 64), __shfl(xe, src, 64), __shfl(xa, src, 64), l, X);
+            row.finish(__shfl(xb, src, 64), __shfl(xe, src, 64), __shfl(xa, src, 64), l, X);
             if constexpr (REFINE) {
 #pragma unroll
                 for (int i = 0; i < E; i++) X[i] = xo[i] + X[i];
@@ -388,7 +478,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         if (threadIdx.x == 0) {
             if (!ok && kind != kFusedHelp) {
                 int& to = kind == kFusedOwn ? head : again;
-                *fused_link(rows, bps, ti) = to;
+                *fw.link(ti) = to;
                 to = tile;
             }
             int t = -1, k = kFusedAgain;
@@ -406,7 +496,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
                     }
                     if (head >= 0) {
                         t = head;
-                        head = *fused_link(loc.Rows(t >> lg_bps), bps, t & (bps - 1));
+                        head = *FusedWords{loc.Rows(t >> lg_bps), bps}.link(t & (bps - 1));
                     }
                 }
                 tries++;
@@ -432,10 +522,10 @@ int resident_workgroups(K kernel, int threads, size_t lds) {
     return cus * occ;
 }
 
-template <bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
+template <int METHOD, bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
 hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, bool* done) {
     const int lg_bps = __builtin_ctz((unsigned)(n / kFusedTile));
-    const auto kern = fused_split_kernel<HAS_B, CT, REFINE, WIDE, Loc>;
+    const auto kern = fused_split_kernel<METHOD, HAS_B, CT, REFINE, WIDE, Loc>;
     // workgroups resident at once, asked once per device: the query costs
     // the host as much as a launch
     static std::atomic<int> known[64];
@@ -453,7 +543,9 @@ hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, b
     if (!*done) return hipSuccess;
     const int tiles = nsys << lg_bps;
     const int grid = tiles < capacity ? tiles : capacity;
-    hipLaunchKernelGGL((clear_fused_kernel<Loc>), dim3((tiles + 255) / 256), dim3(256), 0, stream, loc, nsys, lg_bps);
+    const long long pieces = (long long)nsys * fused_clear_pieces(1 << lg_bps);
+    hipLaunchKernelGGL((clear_fused_kernel<Loc>), dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, loc,
+                       nsys, 1 << lg_bps);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kFusedThreads), 0, stream, loc, nsys, lg_bps, 0, grid, kFusedSpin);
     return hipGetLastError();
 }
@@ -463,10 +555,10 @@ hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, b
 // whole system's workgroups at once (a refinement step on 4 Mi equations, at
 // three workgroups per CU): every tile would be loaded twice (4 Mi equations:
 // 104 us that way, 97 in two passes).
-template <bool HAS_B, typename CT, bool REFINE, typename Loc>
+template <int METHOD, bool HAS_B, typename CT, bool REFINE, typename Loc>
 hipError_t launch_fused(const Loc& loc, int n, int nsys, hipStream_t stream, bool* done) {
-    return n / kFusedTile > kFusedWave ? launch_fused_t<HAS_B, CT, REFINE, true>(loc, n, nsys, stream, done)
-                                       : launch_fused_t<HAS_B, CT, REFINE, false>(loc, n, nsys, stream, done);
+    return n / kFusedTile > kFusedGroup ? launch_fused_t<METHOD, HAS_B, CT, REFINE, true>(loc, n, nsys, stream, done)
+                                       : launch_fused_t<METHOD, HAS_B, CT, REFINE, false>(loc, n, nsys, stream, done);
 }
 
 }  // namespace tprh

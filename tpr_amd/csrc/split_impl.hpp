@@ -7,9 +7,9 @@
 // barriers and limits n to s^2 (src/ptpr.cu:543,581,655).  Here a batch is
 // solved in rounds of `chunk` systems, each round in one of four forms:
 //
-// Fused (split_fused.hpp), the library's form for fast PTPR at s >= 256 (and
+// Fused (split_fused.hpp), the library's form for fast PTPR and TPR at s >= 256 (and
 // what split_form 2 asks for there): one pass over tiles that exchange six
-// numbers each, 65 us for 256 x N=65536.
+// numbers each, 63.5 us for 256 x N=65536.
 //
 // Two passes (split_kernels.hpp), the library's form for everything else:
 //   K1 rows_kernel   : every lane group reduces its slices and writes two
@@ -144,16 +144,16 @@ hipError_t launch_round_pipelined(const SplitArgs& p, size_t base, int cs, int m
     return hipGetLastError();
 }
 
-// The fast one-pass form (split_fused.hpp): s = 256 and more in fast PTPR.
+// The fast one-pass form (split_fused.hpp): s = 256 and more in fast arithmetic.
 template <int METHOD, int MODE>
-constexpr bool kFusedSplit = METHOD == 0 && MODE == kFast;
+constexpr bool kFusedSplit = MODE == kFast;
 
-template <bool HAS_B, typename CT, bool REFINE>
+template <int METHOD, bool HAS_B, typename CT, bool REFINE>
 hipError_t launch_fused_rounds(const SplitArgs& p, int m, hipStream_t stream, bool* done) {
     *done = true;
     for (int s0 = 0; s0 < p.nsys && *done; s0 += p.chunk) {
         const int cs = (p.nsys - s0 < p.chunk) ? p.nsys - s0 : p.chunk;
-        const hipError_t e = launch_fused<HAS_B, CT, REFINE>(round_loc<CT>(p, (size_t)s0 * p.n, m), p.n, cs, stream, done);
+        const hipError_t e = launch_fused<METHOD, HAS_B, CT, REFINE>(round_loc<CT>(p, (size_t)s0 * p.n, m), p.n, cs, stream, done);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -221,14 +221,14 @@ hipError_t launch_split_el(const SplitArgs& p, hipStream_t stream) {
             bool done = false;
             hipError_t e;
             if (p.f16)
-                e = hb ? launch_fused_rounds<true, _Float16, false>(p, m, stream, &done)
-                       : launch_fused_rounds<false, _Float16, false>(p, m, stream, &done);
+                e = hb ? launch_fused_rounds<METHOD, true, _Float16, false>(p, m, stream, &done)
+                       : launch_fused_rounds<METHOD, false, _Float16, false>(p, m, stream, &done);
             else if (p.refine)
-                e = hb ? launch_fused_rounds<true, float, true>(p, m, stream, &done)
-                       : launch_fused_rounds<false, float, true>(p, m, stream, &done);
+                e = hb ? launch_fused_rounds<METHOD, true, float, true>(p, m, stream, &done)
+                       : launch_fused_rounds<METHOD, false, float, true>(p, m, stream, &done);
             else
-                e = hb ? launch_fused_rounds<true, float, false>(p, m, stream, &done)
-                       : launch_fused_rounds<false, float, false>(p, m, stream, &done);
+                e = hb ? launch_fused_rounds<METHOD, true, float, false>(p, m, stream, &done)
+                       : launch_fused_rounds<METHOD, false, float, false>(p, m, stream, &done);
             if (e != hipSuccess || done) return e;
         }
     }

@@ -176,15 +176,15 @@ extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float
     const int lg = __builtin_ctz((unsigned)(n / kFusedTile));
     hipStream_t st = (hipStream_t)stream;
     if (clear) {
-        const int tiles = nsys << lg;
-        hipLaunchKernelGGL((clear_fused_kernel<BatchLoc<float>>), dim3((tiles + 255) / 256), dim3(256), 0, st, loc, nsys,
-                           lg);
+        const int pieces = nsys * fused_clear_pieces(1 << lg);
+        hipLaunchKernelGGL((clear_fused_kernel<BatchLoc<float>>), dim3((pieces + 255) / 256), dim3(256), 0, st, loc,
+                           nsys, 1 << lg);
     }
     const bool wide = (1 << lg) > kFusedWave;
-    auto* kern = refine ? (wide ? fused_split_kernel<true, float, true, true, BatchLoc<float>>
-                                : fused_split_kernel<true, float, true, false, BatchLoc<float>>)
-                        : (wide ? fused_split_kernel<true, float, false, true, BatchLoc<float>>
-                                : fused_split_kernel<true, float, false, false, BatchLoc<float>>);
+    auto* kern = refine ? (wide ? fused_split_kernel<0, true, float, true, true, BatchLoc<float>>
+                                : fused_split_kernel<0, true, float, true, false, BatchLoc<float>>)
+                        : (wide ? fused_split_kernel<0, true, float, false, true, BatchLoc<float>>
+                                : fused_split_kernel<0, true, float, false, false, BatchLoc<float>>);
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), 0, st, loc, nsys, lg, first, stride, spin);
     return (int)hipGetLastError();
 }
