@@ -381,3 +381,41 @@ def test_serve_random_mix_exact(seed):
             srv.matrix_release(m)
         st = srv.stats()
         assert st["failed"] == 0 and st["peak_bytes"] <= budget and st["bytes_in_use"] == 0
+
+
+def test_buffers_of_every_kind_in_one_burst():
+    """Right-hand sides and answers in device memory (16-byte aligned and
+    not), pinned and pageable host memory, in one burst: every answer is the
+    one of a request whose answers stay in the arena, and nothing around the
+    callers' buffers is written."""
+    rng = np.random.default_rng(5)
+    sizes = [(16, 1), (512, 3), (4096, 5), (16384, 2), (32768, 3), (1024, 64)]
+    with Server(512 << 20) as srv:
+        mats = [srv.matrix_generate(n, seed=9, sys=i) for i, (n, _) in enumerate(sizes)]
+        jobs = []
+        for place in ("device", "unaligned", "pinned", "host"):
+            for m, (n, k) in zip(mats, sizes):
+                d = rng.uniform(-1, 1, n * k).astype(np.float32)
+                if place == "host":
+                    x = np.full(n * k + 8, 3.5, np.float32)
+                    jobs.append((m, k, d, d, x[4:4 + n * k], x, 4))
+                    continue
+                kw = {"pin_memory": True} if place == "pinned" else {"device": "cuda"}
+                at = 5 if place == "unaligned" else 4
+                dd = torch.zeros(n * k + 16, **kw)
+                x = torch.full((n * k + 16,), 3.5, **kw)
+                dd[at:at + n * k] = torch.from_numpy(d).to(dd.device)
+                jobs.append((m, k, d, dd[at:at + n * k], x[at:at + n * k], x, at))
+        torch.cuda.synchronize()
+        ids = [srv.submit(m, k, d=d, x=x) for m, k, _, d, x, _, _ in jobs]
+        for r in ids:
+            srv.wait(r)
+        for (m, k, d, _, x, full, at), r in zip(jobs, ids):
+            kept = srv.submit(m, k, d=d)
+            srv.wait(kept)
+            ref = srv.result(kept).cpu().numpy().ravel()
+            srv.release(kept)
+            srv.release(r)
+            out = full.cpu().numpy() if isinstance(full, torch.Tensor) else full
+            assert np.array_equal(out[at:at + ref.size].view(np.int32), ref.view(np.int32)), (at, ref.size)
+            assert (out[:at] == 3.5).all() and (out[at + ref.size:] == 3.5).all()

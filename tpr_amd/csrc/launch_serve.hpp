@@ -15,7 +15,7 @@ namespace tprh {
 struct ServeSys {
     long long coef;  // a at coef, b at coef + n, c at coef + 2n
     long long rhs;   // d
-    long long x;     // answer
+    long long x;     // answer (outside the arena where it goes straight to the caller's buffer)
 };
 
 struct ServeLaunch {
@@ -52,6 +52,23 @@ struct ServeSplitLaunch {
 inline bool serve_split_shape(int E, int L) {
     return (E == 16 && (L == 16 || L == 32 || L == 64)) || (E == 32 && L == 64);
 }
+
+// A copy of `count` floats inside this device's memory; `first`: its first
+// chunk of kCopyChunk floats among all the runs' chunks of a launch.
+constexpr int kCopyChunk = 4096;
+struct CopyRun {
+    const float* src;
+    float* dst;
+    long long count;
+    int first;
+};
+
+// All runs of a device table in one launch (serve_copy.hip), `chunks` chunks
+// in all.  Weak, as is the next: the loop's host code also builds without the
+// kernels (its CPU tests), and then copies run by run.
+__attribute__((weak)) hipError_t launch_copy_runs(const CopyRun* runs, int nruns, int chunks, hipStream_t stream);
+// Whether p lies in memory allocated on `device`; [*lo, *hi): that allocation.
+__attribute__((weak)) bool device_allocation(const void* p, int device, size_t* lo, size_t* hi);
 
 hipError_t launch_serve(int method, int mode, const ServeLaunch& p, hipStream_t stream);
 // The three split kernels over every system of the table (one size class).

@@ -335,6 +335,7 @@ struct Staged {
     int wait_slot;        // generated by another slot's running batch: wait for its generation
     int gen_kind;         // >= 0: this batch generates the matrix (first request to use it)
     uint64_t gen_seed;
+    bool x_direct;        // the solve writes x_dst itself
 };
 
 // Builds and launches one batch on slot `sl` (busy, so this thread owns its
@@ -343,12 +344,14 @@ struct Staged {
 // entries, generation jobs, the serve kernel's zeroed work counter) is
 // packed into the slot's pinned staging buffer and copied with one
 // transfer; then, on the slot's stream: caller right-hand sides are copied
-// in, synthetic ones and the coefficients of matrices first used here are
+// in (those in this device's memory by one kernel), synthetic ones and the coefficients of matrices first used here are
 // generated (one launch, then the gen_done event that batches on other
 // slots using those matrices wait for), the serve kernel runs for every
 // class within a workgroup, one split launch set per larger class, and the
-// answers the caller asked for are copied out.  Returns the first HIP error.
-hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& items) {
+// answers the caller asked for are copied out -- those for 16-byte aligned
+// buffers in this device's memory are written there by the solve itself.
+// Returns the first HIP error.
+hipError_t launch_batch(tprh_server* sv, Slot& sl, std::vector<Staged>& items) {
     float* basef = reinterpret_cast<float*>(sv->base);
     const size_t fsz = sizeof(float);
     hipError_t e = hipSuccess;
@@ -359,7 +362,22 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
     long long gen_total = 0;
     bool generates = false;
     unsigned waited = 0;  // slots already waited for
-    for (const Staged& it : items) {
+    std::vector<tprh::CopyRun> runs;
+    int chunks = 0;
+    // allocations of this device that the batch's buffers were found in (for
+    // this launch only: a caller may free one once its requests are done)
+    std::vector<std::pair<size_t, size_t>> found;
+    auto on_device = [&](const void* p, size_t bytes) {
+        if (!tprh::launch_copy_runs || !tprh::device_allocation) return false;
+        const size_t a = reinterpret_cast<size_t>(p);
+        for (const auto& f : found)
+            if (a >= f.first && a < f.second) return bytes <= f.second - a;
+        size_t lo = 0, hi = 0;
+        if (!tprh::device_allocation(p, sv->device, &lo, &hi)) return false;
+        found.push_back({lo, hi});
+        return a >= lo && a < hi && bytes <= hi - a;
+    };
+    for (Staged& it : items) {
         const Request& r = it.r;
         if (it.ready && (e = hipStreamWaitEvent(sl.stream, it.ready, 0)) != hipSuccess) return e;
         if (it.wait_slot >= 0 && !(waited >> it.wait_slot & 1u)) {
@@ -380,7 +398,11 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
             generates = true;
         }
         const size_t nn = (size_t)r.n;
-        if (r.d_src) {
+        if (r.d_src && on_device(r.d_src, fsz * nn * r.nrhs)) {
+            const long long count = (long long)nn * r.nrhs;
+            runs.push_back({r.d_src, basef + r.off / fsz, count, chunks});
+            chunks += (int)((count + tprh::kCopyChunk - 1) / tprh::kCopyChunk);
+        } else if (r.d_src) {
             if ((e = hipMemcpyAsync(basef + r.off / fsz, r.d_src, fsz * nn * r.nrhs, hipMemcpyDefault, sl.stream)) !=
                 hipSuccess)
                 return e;
@@ -396,6 +418,11 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
             jobs.push_back(jb);
             gen_total += (long long)r.nrhs * r.n;
         }
+        const bool direct = it.x_direct =
+            r.x_dst && (reinterpret_cast<size_t>(r.x_dst) & 15) == 0 && on_device(r.x_dst, fsz * nn * r.nrhs);
+        const long long x_at = direct ? (long long)(reinterpret_cast<intptr_t>(r.x_dst) - reinterpret_cast<intptr_t>(basef)) /
+                                            (long long)fsz
+                                      : (long long)(r.x_off / fsz);
         shape_of[r.n] = {r.E, r.L};
         if (!r.split) {
             auto& g = groups[ClassKey{r.n}];
@@ -403,7 +430,7 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
                 tprh::ServeSys ss;
                 ss.coef = (long long)(it.mat_off / fsz);
                 ss.rhs = (long long)(r.off / fsz + (size_t)j * nn);
-                ss.x = (long long)(r.x_off / fsz + (size_t)j * nn);
+                ss.x = x_at + (long long)((size_t)j * nn);
                 g.push_back(ss);
             }
         } else {
@@ -415,7 +442,7 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
                 tprh::ServeSplitSys ss;
                 ss.coef = (long long)(it.mat_off / fsz);
                 ss.rhs = (long long)(r.off / fsz + (size_t)j * nn);
-                ss.x = (long long)(r.x_off / fsz + (size_t)j * nn);
+                ss.x = x_at + (long long)((size_t)j * nn);
                 ss.rows = (long long)(rows0 + (size_t)j * ms * tprh::kSplitRowWords);
                 ss.xed = (long long)(rows0 + (size_t)r.nrhs * ms * tprh::kSplitRowWords + (size_t)j * ms);
                 g.push_back(ss);
@@ -457,10 +484,14 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
     std::vector<std::pair<size_t, size_t>> split_at;  // (offset, count) per split class, in map order
     for (auto& kv : split_groups)
         split_at.push_back({put(kv.second.data(), sizeof(tprh::ServeSplitSys) * kv.second.size()), kv.second.size()});
+    const size_t o_runs = put(runs.data(), sizeof(tprh::CopyRun) * runs.size());
     const size_t o_jobs = put(jobs.data(), sizeof(tprh::GenJob) * jobs.size());
     const int zero = 0;  // the serve kernel's work counter, cleared by this copy
     const size_t o_counter = tasks.empty() ? 0 : put(&zero, sizeof(int));
     if (at > 0 && (e = hipMemcpyAsync(dt, hs, at, hipMemcpyHostToDevice, sl.stream)) != hipSuccess) return e;
+    if (!runs.empty() && (e = tprh::launch_copy_runs(reinterpret_cast<const tprh::CopyRun*>(dt + o_runs),
+                                                     (int)runs.size(), chunks, sl.stream)) != hipSuccess)
+        return e;
     if (!jobs.empty() &&
         (e = tprh::launch_generate_jobs(reinterpret_cast<const tprh::GenJob*>(dt + o_jobs), (int)jobs.size(),
                                         gen_total, basef, sl.stream)) != hipSuccess)
@@ -492,7 +523,7 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, const std::vector<Staged>& it
     }
     for (const Staged& it : items) {
         const Request& r = it.r;
-        if (r.x_dst &&
+        if (r.x_dst && !it.x_direct &&
             (e = hipMemcpyAsync(r.x_dst, basef + r.x_off / fsz, fsz * (size_t)r.n * r.nrhs, hipMemcpyDefault,
                                 sl.stream)) != hipSuccess)
             return e;
@@ -625,7 +656,7 @@ void worker_main(tprh_server* sv) {
             for (long long id : batch) {
                 const Request& r = sv->reqs[id];
                 Matrix& m = sv->mats[r.mat];
-                Staged it{r, m.off, m.sys, nullptr, -1, -1, 0};
+                Staged it{r, m.off, m.sys, nullptr, -1, -1, 0, false};
                 if (m.ready) {
                     if (!m.ready_known && hipEventQuery(m.ready) == hipSuccess) m.ready_known = true;
                     if (!m.ready_known) it.ready = m.ready;
@@ -778,11 +809,13 @@ tprh_status tprh_server_create(tprh_server** out, const tprh_server_config* cfg)
     // serve kernel's system entries, the split launches' system entries
     // (a batch has at most max_batch_systems right-hand sides, hence at most
     // that many items, entries and requests; split classes add one alignment
-    // pad each, at most 32 of them), the generation jobs (two per request at
-    // most) and the work counter
+    // pad each, at most 32 of them), the copies of right-hand sides (one per
+    // request at most), the generation jobs (two per request at most) and the
+    // work counter
     sv->table_bytes = align_up(sizeof(tprh::UnevenTask) * (size_t)cfg->max_batch_systems) +
                       align_up(sizeof(tprh::ServeSys) * (size_t)cfg->max_batch_systems) +
                       align_up(sizeof(tprh::ServeSplitSys) * (size_t)cfg->max_batch_systems) + 32 * kAlign +
+                      align_up(sizeof(tprh::CopyRun) * (size_t)cfg->max_batch_systems) +
                       align_up(sizeof(tprh::GenJob) * 2 * (size_t)cfg->max_batch_systems) + kAlign;
     sv->slots.resize(cfg->max_inflight);
     for (Slot& sl : sv->slots) {
