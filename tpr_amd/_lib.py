@@ -175,4 +175,5 @@ def check(status, func):
 
 
 def call(name, *args):
-    return check(getattr(lib(), name)(*args), name)
+    status = getattr(_lib or lib(), name)(*args)
+    return status if status == SUCCESS else check(status, name)

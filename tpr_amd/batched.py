@@ -14,24 +14,44 @@ GEN = {"dominant": _lib.GEN_DOMINANT, "weak": _lib.GEN_WEAK, "fixed": _lib.GEN_F
        "random_rhs": _lib.GEN_RANDOM_RHS}
 
 
+torch = None  # the module, once a call has needed it
+
+
+def _torch():
+    global torch
+    if torch is None:
+        import torch as module
+        torch = module
+    return torch
+
+
 def _dptr(t, name, numel=None):
+    """Device address of t (an int, as the library's void* arguments take
+    it).  A small solve is bound by its host calls -- one system of 1024
+    equations takes 4.5 us on the device -- so these helpers look at each
+    tensor once and build no ctypes objects: 9.3 -> 6.0 us a call."""
     if t is None:
         return None
-    import torch
-    if not isinstance(t, torch.Tensor):
+    tt = torch or _torch()
+    if not isinstance(t, tt.Tensor):
         raise TypeError("%s must be a torch tensor" % name)
-    if not t.is_cuda or t.dtype != torch.float32 or not t.is_contiguous():
+    if not t.is_cuda or t.dtype != tt.float32 or not t.is_contiguous():
         raise TypeError("%s must be a contiguous float32 GPU tensor" % name)
     if numel is not None and t.numel() < numel:
         raise ValueError("%s has %d elements, need %d" % (name, t.numel(), numel))
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _stream(stream):
-    import torch
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    """The raw stream: the current one when None.  torch.cuda.current_stream()
+    builds a Stream object (3 us); the raw query is used where torch has it."""
+    if stream is not None:
+        return stream.cuda_stream
+    tt = torch or _torch()
+    raw = getattr(tt._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return tt.cuda.current_stream().cuda_stream
+    return raw(tt.cuda.current_device())
 
 
 def solve_batched(a, b, c, d, x, n, s, method="ptpr", arith="fast", shape=None, stream=None):
@@ -52,12 +72,11 @@ def solve_batched(a, b, c, d, x, n, s, method="ptpr", arith="fast", shape=None, 
     return x
 
 
-def _dptr_any(t, name, numel, dtypes):
-    import torch
+def _dptr_any(t, name, numel, dtype):
     if t is None:
         return None
-    if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous() or t.dtype not in dtypes:
-        raise TypeError("%s must be a contiguous GPU tensor of %s" % (name, dtypes))
+    if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous() or t.dtype != dtype:
+        raise TypeError("%s must be a contiguous GPU tensor of %s" % (name, (dtype,)))
     if t.numel() < numel:
         raise ValueError("%s has %d elements, need %d" % (name, t.numel(), numel))
     return t.data_ptr()
@@ -69,34 +88,29 @@ def make_desc(a, b, c, d, x, n, s, method="ptpr", arith="fast", refine=False, sh
     dtype).  shared: a, b, c hold one matrix (n values) for every right-hand
     side in d.  x_cached: store x through the caches (for a caller whose
     next kernel reads x) instead of non-temporally."""
-    import torch
+    tt = torch or _torch()
     nsys = d.numel() // n
     tot = nsys * n
     ctot = n if shared else tot
-    coef16 = a.dtype == torch.float16
-    cd = (torch.float16,) if coef16 else (torch.float32,)
-    desc = _lib.SolveDesc()
-    desc.method = METHODS[method]
-    desc.arith = ARITH[arith]
-    desc.n, desc.s, desc.nsys = int(n), int(s), int(nsys)
-    desc.coef = _lib.STORE_F16 if coef16 else _lib.STORE_F32
-    desc.a = _dptr_any(a, "a", ctot, cd)
-    desc.b = _dptr_any(b, "b", ctot, cd)
-    desc.c = _dptr_any(c, "c", ctot, cd)
-    desc.d = _dptr_any(d, "d", tot, (torch.float32,))
-    desc.x = _dptr_any(x, "x", tot, (torch.float32,))
-    desc.refine = 1 if refine else 0
-    desc.E, desc.L = shape if shape is not None else (0, 0)
-    desc.chunk = int(chunk)
-    desc.coef_shared = 1 if shared else 0
-    desc.split_form = int(split_form)
-    desc.x_cached = 1 if x_cached else 0
-    return desc
+    coef16 = a.dtype == tt.float16
+    f32 = tt.float32
+    cd = tt.float16 if coef16 else f32
+    E, L = shape if shape is not None else (0, 0)
+    # positional, in the order of SolveDesc's fields (assigning them one by
+    # one takes several times as long)
+    return _lib.SolveDesc(
+        METHODS[method], ARITH[arith], int(n), int(s), int(nsys), _lib.STORE_F16 if coef16 else _lib.STORE_F32,
+        _dptr_any(a, "a", ctot, cd), _dptr_any(b, "b", ctot, cd), _dptr_any(c, "c", ctot, cd),
+        _dptr_any(d, "d", tot, f32), _dptr_any(x, "x", tot, f32), 1 if refine else 0, E, L, int(chunk), None, 0,
+        1 if shared else 0, int(split_form), 1 if x_cached else 0)
+
+
+_NO_SIZE = ctypes.c_size_t(-1).value
 
 
 def workspace_bytes(desc):
     v = _lib.lib().tprh_workspace_bytes(ctypes.byref(desc))
-    if v == ctypes.c_size_t(-1).value:
+    if v == _NO_SIZE:
         _lib.check(_lib.ERROR_INVALID_VALUE, "tprh_workspace_bytes")
     return v
 
@@ -111,7 +125,6 @@ def solve_ex(a, b, c, d, x, n, s, method="ptpr", arith="fast", refine=False, sha
     0 / 1 / 2 / 3: the library's choice / two passes / one pass / pipelined
     for systems above one workgroup; x_cached=True stores x through the
     caches instead of non-temporally (same answers)."""
-    import torch
     desc = make_desc(a, b, c, d, x, n, s, method, arith, refine, shape, chunk, shared, split_form, x_cached)
     need = workspace_bytes(desc)
     own = None

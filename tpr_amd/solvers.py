@@ -37,7 +37,8 @@ def _host_f32(x, name):
 
 
 def _ptr(x):
-    return x.ctypes.data_as(ctypes.c_void_p)
+    # the address alone (x.ctypes builds objects: 1.1 us against 0.5)
+    return x.__array_interface__["data"][0]
 
 
 class _SolverBase:
