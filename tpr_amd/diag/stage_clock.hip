@@ -180,7 +180,7 @@ extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float
         hipLaunchKernelGGL((clear_fused_kernel<BatchLoc<float>>), dim3((pieces + 255) / 256), dim3(256), 0, st, loc,
                            nsys, 1 << lg);
     }
-    const bool wide = (1 << lg) > kFusedWave;
+    const bool wide = (1 << lg) > kFusedGroup;
     auto* kern = refine ? (wide ? fused_split_kernel<0, true, float, true, true, BatchLoc<float>>
                                 : fused_split_kernel<0, true, float, true, false, BatchLoc<float>>)
                         : (wide ? fused_split_kernel<0, true, float, false, true, BatchLoc<float>>
