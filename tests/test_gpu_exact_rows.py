@@ -1,0 +1,107 @@
+"""Exact PTPR with the levels of stage 1 inside the lane (exact_rows.hpp):
+bit identity with the oracle on every shape that runs this way, on inputs
+that reach its corners -- missing partners at the ends of a slice, signed
+zeros, infinities and NaNs beside them, denominators outside the short
+reciprocal's range -- and the short reciprocal itself on every float."""
+import ctypes
+import os
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from tpr_amd import batched as B
+from tpr_amd import build
+
+pytestmark = pytest.mark.gpu
+
+
+def bits_equal(x, y):
+    same = x.view(np.uint32) == y.view(np.uint32)
+    return bool(np.all(same | (np.isnan(x) & np.isnan(y))))
+
+
+def gpu(a, b, c, d, n, s, shape=None, **kw):
+    da, db, dc, dd = (torch.from_numpy(np.ascontiguousarray(v)).cuda() for v in (a, b, c, d))
+    x = torch.full_like(dd, 7.0)
+    B.solve_ex(da, db, dc, dd, x, n, s, arith="exact", shape=shape, **kw)
+    torch.cuda.synchronize()
+    return x.cpu().numpy()
+
+
+SHAPES = [(8, 16), (16, 16), (8, 32), (8, 64), (16, 32), (16, 64), (32, 64)]
+
+
+@pytest.mark.parametrize("E,L", SHAPES)
+@pytest.mark.parametrize("m", [1, 4, 16])
+def test_shapes_bit_identical(E, L, m):
+    s = E * L
+    n = s * m
+    if m * L > 1024:
+        n, m = s * (1024 // L), 1024 // L
+    nsys = 5
+    print("exact rows", E, L, m, flush=True)
+    for kind in (O.GEN_DOMINANT, O.GEN_WEAK):
+        a, b, c, d, _ = O.gen_batch(71, 0, nsys, n, kind)
+        assert bits_equal(gpu(a, b, c, d, n, s, (E, L)), O.solve_batch("ptpr", a, b, c, d, n, s)), kind
+
+
+@pytest.mark.parametrize("E,L", SHAPES)
+def test_special_values_bit_identical(E, L):
+    """One kind of special value per system, spread over every position of a
+    slice: zeros of both signs, infinities, NaN, and off-diagonals that make a
+    denominator zero, subnormal or beyond 2^126."""
+    s = E * L
+    m = 2
+    n = s * m
+    rng = np.random.default_rng(72)
+    special = [(0.0, -0.0), (-0.0, -0.0), (np.inf, 1.0), (np.nan, 0.0), (1e-39, -0.0), (3e38, 0.0), (-1e20, 1e30),
+               (1.0, 1.0)]
+    nsys = len(special)
+    a, b, c, d, _ = O.gen_batch(73, 0, nsys, n, O.GEN_DOMINANT)
+    a, b, c, d = (v.reshape(nsys, n) for v in (a, b, c, d))
+    for k, (off, rhs) in enumerate(special):
+        at = np.unique(np.concatenate([rng.integers(0, n, 12), [0, 1, s - 1, s, n - 2, n - 1]]))
+        b[k] = 1.0
+        for v in (a, c):
+            v[k, at] = np.float32(off)
+        d[k, at[::2]] = np.float32(rhs)
+        if off == 1.0:  # 1 - c a = 0 between neighbours
+            a[k, 1::2], c[k, 0::2] = 1.0, 1.0
+        a[k, 0] = c[k, n - 1] = 0.0
+    a, b, c, d = (np.ascontiguousarray(v.ravel(), np.float32) for v in (a, b, c, d))
+    x = gpu(a, b, c, d, n, s, (E, L)).reshape(nsys, n)
+    with np.errstate(all="ignore"):
+        ref = O.solve_batch("ptpr", a, b, c, d, n, s).reshape(nsys, n)
+    for k in range(nsys):
+        assert bits_equal(x[k], ref[k]), (k, special[k], np.flatnonzero(x[k].view(np.uint32) != ref[k].view(np.uint32))[:8])
+
+
+@pytest.mark.parametrize("n,s", [(32768, 128), (65536, 256), (65536, 1024), (65536, 2048)])
+def test_multi_workgroup_bit_identical(n, s):
+    nsys = 3
+    a, b, c, d, _ = O.gen_batch(74, 0, nsys, n, O.GEN_WEAK)
+    ref = O.solve_batch("ptpr", a, b, c, d, n, s)
+    assert bits_equal(gpu(a, b, c, d, n, s), ref)
+    h = [v.astype(np.float16) for v in (a, b, c)]
+    wide = [v.astype(np.float32) for v in h]
+    assert bits_equal(gpu(*h, d, n, s), O.solve_batch("ptpr", *wide, d, n, s))
+
+
+def test_short_reciprocal_on_every_float():
+    if not os.path.exists(build.DIAG_LIB):
+        pytest.fail("libtpr_diag.so is not built")
+    L = ctypes.CDLL(build.DIAG_LIB)
+    L.tprh_diag_recip_short_check.restype = ctypes.c_int
+    counts = torch.zeros(2, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    print("short reciprocal over 2^32 inputs", flush=True)
+    assert L.tprh_diag_recip_short_check(ctypes.c_void_p(counts.data_ptr()), ctypes.c_void_p(0)) == 0
+    torch.cuda.synchronize()
+    differ, seen = counts.tolist()
+    assert differ == 0
+    # 252 binades of both signs, 2^126 itself, and the NaNs
+    assert seen == 2 * (252 << 23) + 2 + 2 * ((1 << 23) - 1)
+    sys.stdout.flush()

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(BLOCK) void batched_kernel(const CT* __restrict__ a
     float X[E];
     constexpr bool WAVE = BLOCK == kSmallBlock;
     if constexpr (METHOD == 0) {
-        ptpr_solve_raw<E, L, MODE, WAVE>(raw, HAS_B, m, t, my, X);
+        ptpr_solve_raw<E, L, MODE, WAVE, STAGE && kExactTurn<E, L>>(raw, HAS_B, m, t, my, X, stage);
     } else {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, HAS_B, A, C, R);

@@ -21,6 +21,7 @@
 #pragma once
 #include <float.h>
 
+#include "exact_rows.hpp"
 #include "launch.hpp"
 #include "tpr_device.hpp"
 
@@ -705,12 +706,15 @@ __device__ __forceinline__ void tpr_stage3(const float (&A)[E], const float (&C)
 // the same instruction stream on zeros (every lane must take part in the
 // cross-lane exchanges and the barriers) and store nothing.
 // WAVE: the system's lanes lie inside one wavefront (m * L <= 64).
-template <int E, int L, int MODE, bool WAVE = false>
+// TURN: exact stage 1 turned through the wavefront's LDS area `turn`
+// (exact_rows.hpp); X is turned back.
+template <int E, int L, int MODE, bool WAVE = false, bool TURN = false>
 __device__ __forceinline__ void ptpr_solve_regs(float (&A)[E], float (&C)[E], float (&R)[E], int m, int t,
-                                                float* lds, float (&X)[E]) {
+                                                float* lds, float (&X)[E], float* turn = nullptr) {
     const int l = t % L;
     const int j = t / L;
-    ptpr_stage1<E, L, MODE>(A, C, R, l);
+    if constexpr (TURN) exact_stage1_turned<E, L>(A, C, R, l, turn, threadIdx.x & 63);
+    else ptpr_stage1<E, L, MODE>(A, C, R, l);
     if constexpr (WAVE) {
         // the system's lanes are t = 0 .. m L - 1 of one wavefront
         float xe, xprev;
@@ -723,6 +727,7 @@ __device__ __forceinline__ void ptpr_solve_regs(float (&A)[E], float (&C)[E], fl
         const float xprev = (j > 0) ? xr[j - 1] : 0.0f;
         ptpr_stage3<E, L, MODE>(A, C, R, xprev, xr[j], slice_end(lds, m, j), l, X);
     }
+    if constexpr (TURN) turn_blocked<E, L>(X, turn, threadIdx.x & 63);
 }
 
 template <int E, int L, int MODE, bool WAVE = false>
@@ -891,15 +896,17 @@ __device__ __forceinline__ void ptpr_solve_fast16_partition(const RawPart<E>& p,
 // Whole PTPR solve from the raw loads (the division by the diagonal
 // included): the two-level form above where it applies, else the
 // normalisation followed by the register PCR of ptpr_solve_regs.
-template <int E, int L, int MODE, bool WAVE = false>
+// turn: the wavefront's LDS area where the exact form turns its equations
+// (TURN, for the shapes of kExactTurn).
+template <int E, int L, int MODE, bool WAVE = false, bool TURN = false>
 __device__ __forceinline__ void ptpr_solve_raw(const RawPart<E>& raw, bool has_b, int m, int t, float* lds,
-                                               float (&X)[E]) {
+                                               float (&X)[E], float* turn = nullptr) {
     if constexpr (MODE == kFast && L == 16 && E >= 2) {
         ptpr_solve_fast16_partition<E, WAVE>(raw, has_b, m, t, lds, X);
     } else {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, has_b, A, C, R);
-        ptpr_solve_regs<E, L, MODE, WAVE>(A, C, R, m, t, lds, X);
+        ptpr_solve_regs<E, L, MODE, WAVE, TURN && MODE == kExact>(A, C, R, m, t, lds, X, turn);
     }
 }
 

@@ -263,9 +263,12 @@ __global__ __launch_bounds__(256) void stage3_kernel(Loc loc, int lg_m, long lon
     } else if constexpr (METHOD == 0) {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, HAS_B, A, C, R);
-        ptpr_stage1<E, L, MODE>(A, C, R, l);
+        constexpr bool TURN = MODE == kExact && kSplitStaged<E, CT> && kExactTurn<E, L>;
+        if constexpr (TURN) exact_stage1_turned<E, L>(A, C, R, l, stage, threadIdx.x & 63);
+        else ptpr_stage1<E, L, MODE>(A, C, R, l);
         const float* row = rows + (size_t)j * kRowWords;
         ptpr_stage3<E, L, MODE>(A, C, R, xprev, xe, SliceEnd{row[3], row[4], row[5]}, l, X);
+        if constexpr (TURN) turn_blocked<E, L>(X, stage, threadIdx.x & 63);
     } else {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, HAS_B, A, C, R);

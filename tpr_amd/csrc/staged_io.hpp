@@ -19,7 +19,7 @@ namespace tprh {
 
 // The shapes that stage (16-byte pieces of the lanes' runs).
 template <int E>
-constexpr bool kStageX = E == 8 || E == 16;
+constexpr bool kStageX = E == 8 || E == 16 || E == 32;
 
 // The 16-byte pieces of a wavefront's run sit in LDS with one spare slot
 // after every 16 (slot q + q / 16): the per-lane reads and writes of 4 or 2

@@ -9,6 +9,7 @@
 // patterns where the guarded form differs go to bad[].
 #include <hip/hip_runtime.h>
 
+#include "../csrc/exact_rows.hpp"
 #include "../csrc/tpr_device.hpp"
 
 namespace {
@@ -45,7 +46,31 @@ __global__ void recip_check_kernel(unsigned long long* __restrict__ counts, unsi
     if (c4) atomicAdd(&counts[4], c4);
 }
 
+// recip_short (tpr_amd/csrc/exact_rows.hpp) against 1.0f / x for every float
+// with 2^-126 <= |x| <= 2^126 and every NaN: the inputs for which recips_rn
+// takes it.  counts[0]: differences; counts[1]: inputs compared.
+__global__ void recip_short_check_kernel(unsigned long long* __restrict__ counts) {
+    const unsigned long long total = 1ull << 32;
+    const unsigned long long stride = (unsigned long long)gridDim.x * blockDim.x;
+    unsigned long long differ = 0, seen = 0;
+    for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
+        const float x = __builtin_bit_cast(float, (unsigned)i);
+        const float ax = __builtin_fabsf(x);
+        if (x == x && !(ax >= 0x1p-126f && ax <= 0x1p126f)) continue;
+        seen++;
+        if (!same(tprh::recip_short(x), 1.0f / x)) differ++;
+    }
+    if (differ) atomicAdd(&counts[0], differ);
+    atomicAdd(&counts[1], seen);
+}
+
 }  // namespace
+
+// counts: 2 zeroed words.  Returns a hipError_t.
+extern "C" int tprh_diag_recip_short_check(unsigned long long* counts, void* stream) {
+    hipLaunchKernelGGL(recip_short_check_kernel, dim3(8192), dim3(256), 0, (hipStream_t)stream, counts);
+    return (int)hipGetLastError();
+}
 
 // counts: 6 zeroed words (the last one counts recorded patterns); bad: 64
 // words.  Returns a hipError_t.
