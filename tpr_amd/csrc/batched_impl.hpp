@@ -28,6 +28,14 @@ namespace tprh {
 // per wavefront, so the four wavefronts of a workgroup run independently.
 constexpr int kSmallBlock = 256;
 
+// Loads and stores staged through LDS: the shapes of 8, 16 and 32 equations
+// per lane, but for fast TPR on 32 in workgroups of 1024 lanes, whose 128
+// registers a lane the loads in flight then overrun by more (128 systems of
+// N = 32768, s = 2048: 125 us staged, 109 lane by lane; PTPR 125 staged, 143
+// lane by lane).
+template <int METHOD, int E, int MODE, int BLOCK>
+constexpr bool kStageBatched = kStageX<E> && !(METHOD == 1 && MODE == kFast && E == 32 && BLOCK == 1024);
+
 template <int METHOD, int E, int L, int MODE, int BLOCK, bool HAS_B, typename CT, bool REFINE>
 __global__ __launch_bounds__(BLOCK) void batched_kernel(const CT* __restrict__ a, const CT* __restrict__ b,
                                                        const CT* __restrict__ c, const float* __restrict__ d,
@@ -43,7 +51,7 @@ __global__ __launch_bounds__(BLOCK) void batched_kernel(const CT* __restrict__ a
     const size_t off = x0 + (size_t)t * E;
     const size_t coff = shared ? (size_t)t * E : off;  // shared: one matrix for every right-hand side
     // the staged layout: this wavefront's run of 64 E floats and its LDS
-    constexpr bool STAGE = kStageX<E>;
+    constexpr bool STAGE = kStageBatched<METHOD, E, MODE, BLOCK>;
     float* stage = lds + stage_base(blockDim.x >> lg_lanes, m) + (threadIdx.x >> 6) * stage_wave_words<E>();
     const size_t wave_off = ((size_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63)) * E;
     const size_t total = (size_t)nsys * (size_t)n;
@@ -65,11 +73,11 @@ __global__ __launch_bounds__(BLOCK) void batched_kernel(const CT* __restrict__ a
     float X[E];
     constexpr bool WAVE = BLOCK == kSmallBlock;
     if constexpr (METHOD == 0) {
-        ptpr_solve_raw<E, L, MODE, WAVE, STAGE && kExactTurn<E, L>>(raw, HAS_B, m, t, my, X, stage);
+        ptpr_solve_raw<E, L, MODE, WAVE, STAGE && kExactTurn<E, L>>(raw, HAS_B, m, t, my, X, stage, threadIdx.x & 63);
     } else {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, HAS_B, A, C, R);
-        tpr_solve_regs<E, L, MODE, WAVE>(A, C, R, m, t, my, X);
+        tpr_solve_regs<E, L, MODE, WAVE, !(E == 32 && BLOCK == 1024)>(A, C, R, m, t, my, X);
     }
     if constexpr (REFINE) {
 #pragma unroll
@@ -134,7 +142,7 @@ hipError_t launch_el_t(const BatchArgs& p, hipStream_t stream) {
     const int spb = block / T;
     const int grid = (p.nsys + spb - 1) / spb;
     size_t shmem = sizeof(float) * (size_t)spb * lds_words_per_system(p.m);
-    if (kStageX<E>)
+    if (T <= 512 ? kStageX<E> : kStageBatched<METHOD, E, MODE, 1024>)
         shmem = sizeof(float) * ((size_t)stage_base(spb, p.m) + (size_t)stage_words<E>(block));
     // the wavefront-synchronised variant only when a system fits one
     // wavefront; systems of up to 512 lanes take a kernel bounded to 512

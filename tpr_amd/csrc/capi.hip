@@ -489,9 +489,10 @@ tprh_status plan_within(const tprh_solve_desc& d, size_t cap, int* chunk, size_t
 
 // Slice size and shape of the size class n under a 32-row (s, E, L) schedule
 // (NULL or a zero row: s = min(n, 256), default shape).  *split: the class
-// needs the multi-workgroup path.
-tprh_status class_shape(int n, const int* schedule, int* s_out, int* E_out, int* L_out, bool allow_split,
-                        bool* split, int method, int arith) {
+// needs the multi-workgroup path.  nsys: as many systems of this size as
+// would be the caller's work (all of an uneven batch's equations / n).
+tprh_status class_shape_among(int n, int nsys, const int* schedule, int* s_out, int* E_out, int* L_out,
+                              bool allow_split, bool* split, int method, int arith) {
     if (n < 16 || !is_pow2(n)) return fail(TPRH_ERROR_INVALID_VALUE, "system sizes must be powers of two >= 16");
     const int lg = __builtin_ctz((unsigned)n);
     int s = n < 256 ? n : 256, E = 0, L = 0;
@@ -503,10 +504,10 @@ tprh_status class_shape(int n, const int* schedule, int* s_out, int* E_out, int*
         expl = E != 0 || L != 0;
     }
     // exact arithmetic gives the same bits with any shape, so a class without
-    // an explicit shape takes the batched entry's tuned shape for one system
-    // and, where that one has no path in the persistent kernels, the first
+    // an explicit shape takes the batched entry's tuned shape for as many
+    // systems and, where that one has no path in the persistent kernels, the first
     // shape of their menu that fits
-    tprh_status st = check_ns(n, s, 1, &E, &L, expl, allow_split, split,
+    tprh_status st = check_ns(n, s, nsys, &E, &L, expl, allow_split, split,
                               arith == TPRH_ARITH_EXACT ? method : -1, arith);
     if (st != TPRH_SUCCESS) return st;
     if (arith == TPRH_ARITH_EXACT && !expl && !*split && uneven_shape_id(E, L) < 0) {
@@ -526,6 +527,11 @@ tprh_status class_shape(int n, const int* schedule, int* s_out, int* E_out, int*
     return TPRH_SUCCESS;
 }
 
+tprh_status class_shape(int n, const int* schedule, int* s, int* E, int* L, bool allow_split, bool* split, int method,
+                        int arith) {
+    return class_shape_among(n, 1, schedule, s, E, L, allow_split, split, method, arith);
+}
+
 }  // namespace tprh
 
 struct tprh_uneven_plan {
@@ -534,7 +540,7 @@ struct tprh_uneven_plan {
     int nsys = 0;
     int ntasks = 0;
     int grid = 0;
-    size_t lds_bytes = 0;
+    int block = 0;
     long long total = 0;
     std::vector<long long> h_offsets;
     // one device allocation: tasks | sys_list | offsets | sizes | counter
@@ -734,6 +740,8 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
     std::map<int, Cls, std::greater<int>> classes;  // largest systems first
     std::map<int, std::vector<int>> members;
     std::vector<long long> offsets((size_t)nsys + 1, 0);
+    long long equations = 0;  // before the sizes are checked: only a measure of the work
+    for (int k = 0; k < nsys; k++) equations += n[k] > 0 ? n[k] : 0;
     for (int k = 0; k < nsys; k++) {
         const int nk = n[k];
         if (nk < 16 || !is_pow2(nk)) return fail(TPRH_ERROR_INVALID_VALUE, "system sizes must be powers of two >= 16");
@@ -741,7 +749,9 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
         if (!classes.count(nk)) {
             int s = 0, E = 0, L = 0;
             bool split = false;
-            tprh_status st = tprh::class_shape(nk, schedule, &s, &E, &L, false, &split, (int)method, (int)arith);
+            const int among = (int)std::min<long long>(equations / nk, 1 << 30);
+            tprh_status st = tprh::class_shape_among(nk, among, schedule, &s, &E, &L, false, &split, (int)method,
+                                                     (int)arith);
             if (st != TPRH_SUCCESS) return st;
             if (tprh::uneven_shape_id(E, L) < 0)
                 return fail(TPRH_ERROR_NOT_SUPPORTED, "slice shape has no path in the uneven-batch kernel");
@@ -751,11 +761,14 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
     }
     std::vector<tprh::UnevenTask> tasks;
     std::vector<int> sys_list;
-    size_t lds_max = 64;
+    // one workgroup size for the whole plan (launch_uneven.hpp)
+    int lanes = 0;
+    for (const auto& kv : classes) lanes = std::max(lanes, kv.second.m * kv.second.L);
+    const int block = tprh::slot_block(lanes);
     for (const auto& kv : classes) {
         const Cls& c = kv.second;
         const int T = c.m * c.L;
-        const int per = 1024 / T;
+        const int per = block / T;
         const std::vector<int>& mem = members[kv.first];
         for (size_t i = 0; i < mem.size(); i += per) {
             tprh::UnevenTask tk;
@@ -767,7 +780,6 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
             for (int q = 0; q < tk.count; q++) sys_list.push_back(mem[i + q]);
             tasks.push_back(tk);
         }
-        lds_max = std::max(lds_max, sizeof(float) * (size_t)per * tprh::lds_words_per_system(c.m));
     }
     tprh_uneven_plan* pl = new (std::nothrow) tprh_uneven_plan();
     if (!pl) return fail(TPRH_ERROR_OUT_OF_MEMORY, "plan allocation");
@@ -775,7 +787,7 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
     pl->arith = arith;
     pl->nsys = nsys;
     pl->ntasks = (int)tasks.size();
-    pl->lds_bytes = lds_max;
+    pl->block = block;
     pl->total = offsets[nsys];
     pl->h_offsets = offsets;
     const size_t bt = sizeof(tprh::UnevenTask) * tasks.size();
@@ -807,7 +819,7 @@ tprh_status tprh_uneven_plan_create(tprh_uneven_plan** out, tprh_method method, 
     int dev = 0, cus = 0, occ = 0;
     if ((e = hipGetDevice(&dev)) != hipSuccess ||
         (e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess ||
-        (e = tprh::uneven_occupancy(method == TPRH_PTPR ? 0 : 1, arith == TPRH_ARITH_EXACT ? 1 : 0, lds_max, &occ)) !=
+        (e = tprh::uneven_occupancy(method == TPRH_PTPR ? 0 : 1, arith == TPRH_ARITH_EXACT ? 1 : 0, &occ)) !=
             hipSuccess) {
         (void)hipFree(pl->dev);
         delete pl;
@@ -824,8 +836,8 @@ tprh_status tprh_uneven_solve(const tprh_uneven_plan* plan, const float* a, cons
     if (!plan) return fail(TPRH_ERROR_INVALID_VALUE, "null plan");
     if (plan->ntasks == 0) return TPRH_SUCCESS;
     if (!a || !c || !d || !x) return fail(TPRH_ERROR_INVALID_VALUE, "null array pointer");
-    tprh::UnevenLaunch p{plan->tasks, plan->ntasks, plan->counter, plan->sys_list, plan->offsets, a, b, c, d, x,
-                         plan->grid, plan->lds_bytes};
+    tprh::UnevenLaunch p{plan->tasks, plan->ntasks, plan->block, plan->counter, plan->sys_list, plan->offsets, a, b, c, d, x,
+                         plan->grid};
     hipError_t e = tprh::launch_uneven(plan->method == TPRH_PTPR ? 0 : 1, plan->arith == TPRH_ARITH_EXACT ? 1 : 0, p,
                                        (hipStream_t)stream);
     if (e != hipSuccess) return fail_hip(e, "uneven kernel launch");

@@ -128,13 +128,6 @@ __device__ __forceinline__ float exact_keep_dn(float s, float u, int l) {
     }
 }
 
-// v, computed here: the compiler otherwise leaves a level's sums until after
-// its reciprocals and holds their products instead, twice the registers.
-__device__ __forceinline__ float settled(float v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 // x[k] -> 1 / x[k], rounded as IEEE division does: the short sequence of
 // recip_rn without its fixup, which equals division for every |x| in
 // [2^-126, 2^126] and for NaN (checked on every float by

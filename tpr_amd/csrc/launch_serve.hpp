@@ -21,12 +21,12 @@ struct ServeSys {
 struct ServeLaunch {
     const UnevenTask* tasks;  // work items (the shape ids of launch_uneven.hpp)
     int ntasks;
+    int block;     // lanes of a workgroup
     int* counter;  // work counter: must hold 0 when the launch starts (the
                    // serving loop's table copy writes it, no launch of its own)
     const ServeSys* sys;
     float* base;  // arena base
-    int grid;
-    size_t lds_bytes;
+    int grid;     // workgroups of the persistent kernel
 };
 
 // A system of a serving batch whose class needs the multi-workgroup path:

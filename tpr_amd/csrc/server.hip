@@ -216,7 +216,6 @@ struct tprh_server {
     std::vector<Slot> slots;
     hipStream_t upload = nullptr;
     int grid = 1;
-    size_t lds_bytes = 0;
     size_t table_bytes = 0;  // capacity of a slot's packed tables (the work counter included)
     std::thread worker;
     bool stop = false;
@@ -238,10 +237,6 @@ struct tprh_server {
 };
 
 namespace {
-
-// LDS of the serve kernel: a work item holds 1024 / (m L) systems of 13 m
-// floats each, at most 13 * 1024 / 16 floats for any shape of the menu.
-constexpr size_t kServeLds = sizeof(float) * 13 * 1024 / 16;
 
 void free_matrix_locked(tprh_server* sv, long long id) {
     auto it = sv->mats.find(id);
@@ -451,12 +446,17 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, std::vector<Staged>& items) {
     }
     std::vector<tprh::UnevenTask> tasks;
     std::vector<tprh::ServeSys> entries;
+    // one workgroup size for the whole batch (launch_uneven.hpp)
+    int lanes = 0;
+    for (auto& kv : groups)
+        lanes = std::max(lanes, kv.first.n / shape_of[kv.first.n].first);
+    const int block = tprh::slot_block(lanes);
     for (auto& kv : groups) {
         const int n = kv.first.n;
         const int E = shape_of[n].first, L = shape_of[n].second;
         const int m = n / (E * L);
         const int T = m * L;
-        const int per = 1024 / T;
+        const int per = block / T;
         const std::vector<tprh::ServeSys>& v = kv.second;
         for (size_t i = 0; i < v.size(); i += per) {
             tprh::UnevenTask tk;
@@ -502,11 +502,11 @@ hipError_t launch_batch(tprh_server* sv, Slot& sl, std::vector<Staged>& items) {
         tprh::ServeLaunch p;
         p.tasks = reinterpret_cast<const tprh::UnevenTask*>(dt + o_tasks);
         p.ntasks = (int)tasks.size();
+        p.block = block;
         p.counter = reinterpret_cast<int*>(dt + o_counter);
         p.sys = reinterpret_cast<const tprh::ServeSys*>(dt + o_entries);
         p.base = basef;
         p.grid = std::max(1, std::min(sv->grid, p.ntasks));
-        p.lds_bytes = sv->lds_bytes;
         if ((e = tprh::launch_serve(sv->method, sv->mode, p, sl.stream)) != hipSuccess) return e;
     }
     size_t k = 0;
@@ -841,9 +841,8 @@ tprh_status tprh_server_create(tprh_server** out, const tprh_server_config* cfg)
         if ((e = hipStreamSynchronize(sl.stream)) != hipSuccess) return bail(e, "hipStreamSynchronize");
     }
     int cus = 0, occ = 0;
-    sv->lds_bytes = kServeLds;
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, sv->device)) != hipSuccess ||
-        (e = tprh::serve_occupancy(sv->method, sv->mode, sv->lds_bytes, &occ)) != hipSuccess)
+        (e = tprh::serve_occupancy(sv->method, sv->mode, tprh::slot_big_lds(sv->method, sv->mode), &occ)) != hipSuccess)
         return bail(e, "device query");
     sv->grid = std::max(1, cus * std::max(1, occ));
     sv->st.budget = cfg->hbm_budget;

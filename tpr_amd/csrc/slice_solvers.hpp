@@ -316,7 +316,9 @@ __device__ __forceinline__ void ptpr_stage1_fast16(float (&Ap)[E], float (&Cp)[E
 // original values in Ao/Co/Ro for stage 3 (the reference's bkup of
 // src/tpr.cpp:128-132); odd offsets end with their stage-1 values
 // (src/tpr.cpp:209-213).
-template <int E, int L, int MODE, int U>
+// SETTLE: see settled(); not where a lane's 128 registers overflow either way
+// (E = 32 in workgroups of 1024 lanes spills 1756 bytes with it, 596 without).
+template <int E, int L, int MODE, int U, bool SETTLE = true>
 __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], float (&R)[E], int l) {
     constexpr int S = E * L;
     constexpr int P = 2 * U;
@@ -342,7 +344,7 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
                 Eq kl = (j >= U) ? Eq{A[j - U], C[j - U], R[j - U]} : left;
                 Eq kr{A[j + U], C[j + U], R[j + U]};
                 bool hasL = (j >= U) || (l > 0);
-                Eq o = pcr_update<MODE>(Eq{A[j], C[j], R[j]}, kl, kr, hasL, true);
+                Eq o = pcr_update<MODE, SETTLE>(Eq{A[j], C[j], R[j]}, kl, kr, hasL, true);
                 nA[j] = o.a;
                 nC[j] = o.c;
                 nR[j] = o.r;
@@ -353,7 +355,7 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
                 Eq kl{A[k - U], C[k - U], R[k - U]};
                 Eq kr = (k + U < E) ? Eq{A[k + U], C[k + U], R[k + U]} : right;
                 bool hasR = (k + U < E) || (l < L - 1);
-                Eq o = pcr_update<MODE>(Eq{A[k], C[k], R[k]}, kl, kr, true, hasR);
+                Eq o = pcr_update<MODE, SETTLE>(Eq{A[k], C[k], R[k]}, kl, kr, true, hasR);
                 nA[k] = o.a;
                 nC[k] = o.c;
                 nR[k] = o.r;
@@ -382,8 +384,8 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
         Eq el{shift_up<L, D>(e0.a, -1.0f, l), shift_up<L, D>(e0.c, 0.0f, l), shift_up<L, D>(e0.r, 0.0f, l)};
         Eq er{shift_down<L, D>(e0.a, 0.0f, l), shift_down<L, D>(e0.c, -1.0f, l),
               shift_down<L, D>(e0.r, 0.0f, l)};
-        Eq so = pcr_update<MODE>(s0, sl, sr, hasL, hasR);
-        Eq eo = pcr_update<MODE>(e0, el, er, hasL, hasR);
+        Eq so = pcr_update<MODE, SETTLE>(s0, sl, sr, hasL, hasR);
+        Eq eo = pcr_update<MODE, SETTLE>(e0, el, er, hasL, hasR);
         if (lq == 0) {
             A[0] = so.a;
             C[0] = so.c;
@@ -395,7 +397,7 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
             R[E - 1] = eo.r;
         }
     }
-    if constexpr (P < S) tpr_stage1_level<E, L, MODE, P>(A, C, R, l);
+    if constexpr (P < S) tpr_stage1_level<E, L, MODE, P, SETTLE>(A, C, R, l);
 }
 
 // TPR stage 3 (src/tpr.cpp:277-308): tree back-substitution.  X[E-1] of the
@@ -707,13 +709,14 @@ __device__ __forceinline__ void tpr_stage3(const float (&A)[E], const float (&C)
 // cross-lane exchanges and the barriers) and store nothing.
 // WAVE: the system's lanes lie inside one wavefront (m * L <= 64).
 // TURN: exact stage 1 turned through the wavefront's LDS area `turn`
-// (exact_rows.hpp); X is turned back.
+// (exact_rows.hpp; lane: the lane's number in the wavefront); X is turned
+// back.
 template <int E, int L, int MODE, bool WAVE = false, bool TURN = false>
 __device__ __forceinline__ void ptpr_solve_regs(float (&A)[E], float (&C)[E], float (&R)[E], int m, int t,
-                                                float* lds, float (&X)[E], float* turn = nullptr) {
+                                                float* lds, float (&X)[E], float* turn = nullptr, int lane = 0) {
     const int l = t % L;
     const int j = t / L;
-    if constexpr (TURN) exact_stage1_turned<E, L>(A, C, R, l, turn, threadIdx.x & 63);
+    if constexpr (TURN) exact_stage1_turned<E, L>(A, C, R, l, turn, lane);
     else ptpr_stage1<E, L, MODE>(A, C, R, l);
     if constexpr (WAVE) {
         // the system's lanes are t = 0 .. m L - 1 of one wavefront
@@ -727,10 +730,10 @@ __device__ __forceinline__ void ptpr_solve_regs(float (&A)[E], float (&C)[E], fl
         const float xprev = (j > 0) ? xr[j - 1] : 0.0f;
         ptpr_stage3<E, L, MODE>(A, C, R, xprev, xr[j], slice_end(lds, m, j), l, X);
     }
-    if constexpr (TURN) turn_blocked<E, L>(X, turn, threadIdx.x & 63);
+    if constexpr (TURN) turn_blocked<E, L>(X, turn, lane);
 }
 
-template <int E, int L, int MODE, bool WAVE = false>
+template <int E, int L, int MODE, bool WAVE = false, bool SETTLE = true>
 __device__ __forceinline__ void tpr_solve_regs(float (&A)[E], float (&C)[E], float (&R)[E], int m, int t,
                                                float* lds, float (&X)[E]) {
     const int l = t % L;
@@ -742,7 +745,7 @@ __device__ __forceinline__ void tpr_solve_regs(float (&A)[E], float (&C)[E], flo
         Co[i] = C[i];
         Ro[i] = R[i];
     }
-    tpr_stage1_level<E, L, MODE, 1>(A, C, R, l);
+    tpr_stage1_level<E, L, MODE, 1, SETTLE>(A, C, R, l);
     if constexpr (WAVE) {
         // the system's lanes are t = 0 .. m L - 1 of one wavefront
         float xe, xprev;
@@ -900,13 +903,13 @@ __device__ __forceinline__ void ptpr_solve_fast16_partition(const RawPart<E>& p,
 // (TURN, for the shapes of kExactTurn).
 template <int E, int L, int MODE, bool WAVE = false, bool TURN = false>
 __device__ __forceinline__ void ptpr_solve_raw(const RawPart<E>& raw, bool has_b, int m, int t, float* lds,
-                                               float (&X)[E], float* turn = nullptr) {
+                                               float (&X)[E], float* turn = nullptr, int lane = 0) {
     if constexpr (MODE == kFast && L == 16 && E >= 2) {
         ptpr_solve_fast16_partition<E, WAVE>(raw, has_b, m, t, lds, X);
     } else {
         float A[E], C[E], R[E];
         normalise<E, MODE>(raw, has_b, A, C, R);
-        ptpr_solve_regs<E, L, MODE, WAVE, TURN && MODE == kExact>(A, C, R, m, t, lds, X, turn);
+        ptpr_solve_regs<E, L, MODE, WAVE, TURN && MODE == kExact>(A, C, R, m, t, lds, X, turn, lane);
     }
 }
 
