@@ -105,3 +105,51 @@ def test_short_reciprocal_on_every_float():
     # 252 binades of both signs, 2^126 itself, and the NaNs
     assert seen == 2 * (252 << 23) + 2 + 2 * ((1 << 23) - 1)
     sys.stdout.flush()
+
+
+def diag(name):
+    if not os.path.exists(build.DIAG_LIB):
+        pytest.fail("libtpr_diag.so is not built")
+    f = getattr(ctypes.CDLL(build.DIAG_LIB), name)
+    f.restype = ctypes.c_int
+    return f
+
+
+def test_short_quotient():
+    """n / x for 4096 significands of x, the ends of their range among them,
+    against every significand of n."""
+    counts = torch.zeros(2, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    f = diag("tprh_diag_quot_short_check")
+    for first, stride, blocks in ((0, 1, 512), ((1 << 23) - 512, 1, 512), (1777, 2729, 3072)):
+        print("short quotient", first, stride, blocks, flush=True)
+        assert f(blocks, ctypes.c_uint(first), ctypes.c_uint(stride), ctypes.c_void_p(counts.data_ptr()),
+                 ctypes.c_void_p(0)) == 0
+        torch.cuda.synchronize()
+    assert counts.tolist() == [0, 4096 << 23]
+
+
+@pytest.mark.parametrize("kind", ["plain", "zeros", "range", "special"])
+def test_quotients_of_one_divisor(kind):
+    """Whole wavefronts on the short path, and ones that zeros, values at and
+    past the ends of its range, infinities and NaNs send to division or not."""
+    rng = np.random.default_rng(75)
+    blocks = 64
+    v = rng.uniform(0.5, 2.0, (blocks, 4, 64, 8)) * rng.choice([-1.0, 1.0], (blocks, 4, 64, 8))
+    v = v.astype(np.float32)
+    odd = {"plain": [], "zeros": [0.0, -0.0],
+           "range": [2.0**-60, np.nextafter(np.float32(2.0**-60), np.float32(0)), 2.0**60,
+                     np.nextafter(np.float32(2.0**60), np.float32(np.inf)), 1e-40, -1e-45, 3e38, -2.0**-100],
+           "special": [np.inf, -np.inf, np.nan, 0.0, -0.0]}[kind]
+    if odd:
+        # the first half of the workgroups in a, c, d alone, the rest in b too
+        hit = rng.random(v.shape) < 0.02
+        hit[: blocks // 2, 3] = False
+        v[hit] = rng.choice(np.array(odd, np.float32), int(hit.sum()))
+    counts = torch.zeros(2, dtype=torch.int64, device="cuda")
+    ops = torch.from_numpy(np.ascontiguousarray(v)).cuda()
+    torch.cuda.synchronize()
+    assert diag("tprh_diag_quots_check")(ctypes.c_void_p(ops.data_ptr()), blocks, ctypes.c_void_p(counts.data_ptr()),
+                                         ctypes.c_void_p(0)) == 0
+    torch.cuda.synchronize()
+    assert counts.tolist() == [0, blocks * 64 * 24]

@@ -72,12 +72,16 @@ __global__ __launch_bounds__(BLOCK) void batched_kernel(const CT* __restrict__ a
     }
     float X[E];
     constexpr bool WAVE = BLOCK == kSmallBlock;
+    // 32 equations per lane overflow the 128 registers of a 1024-lane
+    // workgroup: what saves registers or time elsewhere adds spills there
+    // (PTPR with quots_rn 4804 bytes per lane, without 940)
+    constexpr bool FITS = !(E == 32 && BLOCK == 1024);
     if constexpr (METHOD == 0) {
-        ptpr_solve_raw<E, L, MODE, WAVE, STAGE && kExactTurn<E, L>>(raw, HAS_B, m, t, my, X, stage, threadIdx.x & 63);
+        ptpr_solve_raw<E, L, MODE, WAVE, STAGE && kExactTurn<E, L>, FITS>(raw, HAS_B, m, t, my, X, stage, threadIdx.x & 63);
     } else {
         float A[E], C[E], R[E];
-        normalise<E, MODE>(raw, HAS_B, A, C, R);
-        tpr_solve_regs<E, L, MODE, WAVE, !(E == 32 && BLOCK == 1024)>(A, C, R, m, t, my, X);
+        normalise<E, MODE, FITS>(raw, HAS_B, A, C, R);
+        tpr_solve_regs<E, L, MODE, WAVE, FITS>(A, C, R, m, t, my, X);
     }
     if constexpr (REFINE) {
 #pragma unroll

@@ -5,7 +5,8 @@
 // operations as they are: at each of log2 S levels every equation takes nine
 // products, four sums and an IEEE reciprocal, none of them fused.  For
 // 4096 x N=1024 the instructions left here take 21 us to issue (2450 and 170
-// reciprocal seeds per wavefront, at 4 and 16 cycles), its memory traffic 14.
+// reciprocal seeds per wavefront, at 4 and 16 cycles; 18 with quots_rn), its
+// memory traffic 14.
 // So what can be saved is everything else: exchanges between lanes, selects
 // for missing partners, and the guard and branch of each reciprocal.
 //
@@ -24,11 +25,12 @@
 // selects: the fused DPP products leave the lanes without a partner alone.
 // A level's reciprocals share one range test and one wave-uniform branch.
 //
-// Measured (fp32 with a diagonal; the register form before -> this form),
-// 4096 systems of N = 1024: 16 x 16 42.5 -> 28.1 us (8 x 32 39.2 -> 32.4,
-// 4 x 64, which stays in registers, 34.8), 16 x 32 50.4 -> 31.2, 8 x 64 41.9
-// -> 34.2; 512 of N = 8192, S = 2048 (32 x 64) 111 -> 38.5.  One system of
-// N = 1024: 8 x 32 10.8 -> 7.1, 4 x 64 6.9.
+// Measured (fp32 with a diagonal; the register form before -> this form ->
+// with the quotients of quots_rn), 4096 systems of N = 1024: 16 x 16 42.5 ->
+// 28.1 -> 25.4 us (8 x 32 39.2 -> 32.4, 4 x 64, which stays in registers,
+// 34.8), 16 x 32 50.4 -> 31.2, 8 x 64 41.9 -> 34.2; 512 of N = 8192, S = 2048
+// (32 x 64) 111 -> 38.5.  One system of N = 1024: 8 x 32 10.8 -> 7.1 -> 6.9,
+// 4 x 64 7.0.  Exact TPR, which divides alike, 20.5 -> 18.6 on the 4096.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -154,6 +156,65 @@ __device__ __forceinline__ void recips_rn(float (&x)[E]) {
         for (int k = 0; k < E; k++) {
             x[k] = 1.0f / x[k];
             __builtin_amdgcn_sched_barrier(0);  // one at a time: this path must not set the register count
+        }
+    }
+}
+
+// Equations that quots_rn puts behind one branch.  All 16 at once: 139
+// registers in place of 129 (split_kernels.hpp, stage 3 of 16 x 16), and 256
+// in place of 233 on 32 equations per lane.
+constexpr int kQuotChunk = 8;
+
+// n / x for y = recip_short(x), rounded as IEEE division does, where n is zero
+// or |n| and |x| lie in [2^-60, 2^60].  y is then 1 / x rounded to nearest,
+// and one correction of n y rounds the quotient right: so for every pair of
+// significands (all 2^46 compared with n / x; the powers of two only scale,
+// nothing here being subnormal or infinite).  The fixup keeps the sign of a
+// zero and the results of infinities and NaNs.
+__device__ __forceinline__ float quot_short(float n, float x, float y) {
+    const float q = n * y;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-x, q, n), y, q), x, n);
+}
+
+// a[k], c[k], d[k] -> their quotients by b[k], rounded as IEEE division does
+// (src/ptpr.hpp:80-90): three quotients of one reciprocal, 25 issue slots per
+// equation against 42 for three divisions, range tests included.  Eight
+// equations at a time share one branch for the wavefront.
+template <int E>
+__device__ __forceinline__ void quots_rn(const float (&a)[E], const float (&c)[E], const float (&d)[E],
+                                         const float (&b)[E], float (&A)[E], float (&C)[E], float (&R)[E]) {
+    constexpr int W = E < kQuotChunk ? E : kQuotChunk;
+    // 2 |v| as a bit pattern, a zero above all others
+    auto key = [](float v) { return (__builtin_bit_cast(unsigned, v) << 1) - 1u; };
+    auto least = [](unsigned u, unsigned v) { return u < v ? u : v; };
+#pragma unroll
+    for (int k0 = 0; k0 < E; k0 += W) {
+        float mx = 0.0f, bn = __builtin_fabsf(b[k0]);
+        unsigned kn = 0xffffffffu;
+#pragma unroll
+        for (int k = k0; k < k0 + W; k++) {
+            mx = __builtin_fmaxf(__builtin_fmaxf(mx, __builtin_fabsf(a[k])), __builtin_fabsf(c[k]));
+            mx = __builtin_fmaxf(__builtin_fmaxf(mx, __builtin_fabsf(d[k])), __builtin_fabsf(b[k]));
+            bn = __builtin_fminf(bn, __builtin_fabsf(b[k]));
+            kn = least(kn, least(key(a[k]), least(key(c[k]), key(d[k]))));
+        }
+        const bool plain = mx <= 0x1p60f && bn >= 0x1p-60f && kn >= key(0x1p-60f);
+        if (__ballot(!plain) == 0) {
+#pragma unroll
+            for (int k = k0; k < k0 + W; k++) {
+                const float y = recip_short(b[k]);
+                A[k] = quot_short(a[k], b[k], y);
+                C[k] = quot_short(c[k], b[k], y);
+                R[k] = quot_short(d[k], b[k], y);
+            }
+        } else {
+#pragma unroll
+            for (int k = k0; k < k0 + W; k++) {
+                A[k] = a[k] / b[k];
+                C[k] = c[k] / b[k];
+                R[k] = d[k] / b[k];
+                __builtin_amdgcn_sched_barrier(0);  // one at a time: this path must not set the register count
+            }
         }
     }
 }

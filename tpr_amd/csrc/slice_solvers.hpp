@@ -163,22 +163,27 @@ __device__ __forceinline__ void load_x_with_halo(const float* __restrict__ x, si
 
 // Divides by the diagonal as the 4-argument setter does (src/ptpr.hpp:80-90);
 // has_b == false means a unit diagonal (the reference's GPU entry points).
-template <int E, int MODE>
+// SHORT: exact quotients by quots_rn.
+template <int E, int MODE, bool SHORT = true>
 __device__ __forceinline__ void normalise(const RawPart<E>& p, bool has_b, float (&A)[E], float (&C)[E],
                                           float (&R)[E]) {
+    if constexpr (MODE == kExact) {
+        if (SHORT && has_b) {
+            quots_rn<E>(p.a, p.c, p.d, p.b, A, C, R);
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < E; i++) {
-        if (has_b) {
-            if constexpr (MODE == kExact) {
-                A[i] = p.a[i] / p.b[i];
-                C[i] = p.c[i] / p.b[i];
-                R[i] = p.d[i] / p.b[i];
-            } else {
-                const float rb = fast_rcp(p.b[i]);
-                A[i] = p.a[i] * rb;
-                C[i] = p.c[i] * rb;
-                R[i] = p.d[i] * rb;
-            }
+        if (MODE == kExact && has_b) {
+            A[i] = p.a[i] / p.b[i];
+            C[i] = p.c[i] / p.b[i];
+            R[i] = p.d[i] / p.b[i];
+        } else if (has_b) {
+            const float rb = fast_rcp(p.b[i]);
+            A[i] = p.a[i] * rb;
+            C[i] = p.c[i] * rb;
+            R[i] = p.d[i] * rb;
         } else {
             A[i] = p.a[i];
             C[i] = p.c[i];
@@ -901,14 +906,14 @@ __device__ __forceinline__ void ptpr_solve_fast16_partition(const RawPart<E>& p,
 // normalisation followed by the register PCR of ptpr_solve_regs.
 // turn: the wavefront's LDS area where the exact form turns its equations
 // (TURN, for the shapes of kExactTurn).
-template <int E, int L, int MODE, bool WAVE = false, bool TURN = false>
+template <int E, int L, int MODE, bool WAVE = false, bool TURN = false, bool SHORT = true>
 __device__ __forceinline__ void ptpr_solve_raw(const RawPart<E>& raw, bool has_b, int m, int t, float* lds,
                                                float (&X)[E], float* turn = nullptr, int lane = 0) {
     if constexpr (MODE == kFast && L == 16 && E >= 2) {
         ptpr_solve_fast16_partition<E, WAVE>(raw, has_b, m, t, lds, X);
     } else {
         float A[E], C[E], R[E];
-        normalise<E, MODE>(raw, has_b, A, C, R);
+        normalise<E, MODE, SHORT>(raw, has_b, A, C, R);
         ptpr_solve_regs<E, L, MODE, WAVE, TURN && MODE == kExact>(A, C, R, m, t, lds, X, turn, lane);
     }
 }

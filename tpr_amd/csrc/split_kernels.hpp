@@ -57,6 +57,11 @@ __device__ __forceinline__ void slice_index(long long gs, int lg_m, int l, long 
 template <int METHOD, int E, int L, int MODE>
 constexpr bool kSplitTwoLevel = METHOD == 0 && MODE == kFast && L == 16 && E >= 2;
 
+// Exact kernels of up to 16 equations per lane are kept to the 128 registers
+// that four wavefronts per SIMD leave; they need a few more otherwise.
+template <int E, int MODE>
+constexpr int kExactWaves = MODE == kExact && E <= 16 ? 4 : 1;
+
 // K1 and K3 load (and K3 stores) their slices as 1 KB runs per instruction
 // through LDS (staged_io.hpp) where the shape stages: a wavefront holds 64 / L whole slices of one system (m L > 1024), one
 // contiguous run starting at `run`.  256-lane workgroups: four wavefronts.
@@ -79,7 +84,7 @@ __device__ __forceinline__ void load_slices(const Loc& loc, long long q, size_t 
 }
 
 template <int METHOD, int E, int L, int MODE, bool HAS_B, typename CT, bool REFINE, typename Loc>
-__global__ __launch_bounds__(256) void rows_kernel(Loc loc, int lg_m, long long nslices) {
+__global__ __launch_bounds__(256, (kExactWaves<E, MODE>)) void rows_kernel(Loc loc, int lg_m, long long nslices) {
     __shared__ __align__(16) float stage_lds[kSplitStageWords<E, CT>];
     const int l = threadIdx.x % L;
     const long long g = (long long)blockIdx.x * (blockDim.x / L) + threadIdx.x / L;  // slice over the round
@@ -216,7 +221,7 @@ __global__ __launch_bounds__(1024) void reduced_kernel(Loc loc) {
 }
 
 template <int METHOD, int E, int L, int MODE, bool HAS_B, typename CT, bool REFINE, typename Loc>
-__global__ __launch_bounds__(256) void stage3_kernel(Loc loc, int lg_m, long long nslices) {
+__global__ __launch_bounds__(256, (kExactWaves<E, MODE>)) void stage3_kernel(Loc loc, int lg_m, long long nslices) {
     __shared__ __align__(16) float stage_lds[kSplitStageWords<E, CT>];
     const int l = threadIdx.x % L;
     // workgroups take the slices in the reverse of K1's order: the slices K1

@@ -64,7 +64,56 @@ __global__ void recip_short_check_kernel(unsigned long long* __restrict__ counts
     atomicAdd(&counts[1], seen);
 }
 
+// quot_short against n / x: `blocks` workgroups, workgroup k with the
+// significand first + k * stride of x, all 2^23 of n, at random powers of two
+// that keep both inside [2^-60, 2^60], and both signs.  counts[0]:
+// differences; counts[1]: pairs compared.
+__global__ void quot_short_check_kernel(unsigned first, unsigned stride, unsigned long long* __restrict__ counts) {
+    const unsigned sx = (first + blockIdx.x * stride) & 0x7fffffu;
+    unsigned long long differ = 0, seen = 0;
+    unsigned rnd = sx * 2654435761u + threadIdx.x * 40503u + 12345u;
+    for (unsigned sn = threadIdx.x; sn < (1u << 23); sn += blockDim.x) {
+        rnd = rnd * 1664525u + 1013904223u;
+        const unsigned ex = 67 + (rnd >> 8) % 120, en = 67 + (rnd >> 16) % 120;  // 2^-60 .. 2^59
+        const float x = __builtin_bit_cast(float, (rnd & 0x80000000u) | ex << 23 | sx);
+        const float n = __builtin_bit_cast(float, (rnd << 1 & 0x80000000u) | en << 23 | sn);
+        seen++;
+        if (!same(tprh::quot_short(n, x, tprh::recip_short(x)), n / x)) differ++;
+    }
+    if (differ) atomicAdd(&counts[0], differ);
+    atomicAdd(&counts[1], seen);
+}
+
+// quots_rn against the division of its operands, one lane's eight equations:
+// ops holds 4 x 8 x 64 floats per workgroup (a, c, d, b of 64 lanes by 8).
+__global__ void quots_check_kernel(const float* __restrict__ ops, unsigned long long* __restrict__ counts) {
+    const float* p = ops + (size_t)blockIdx.x * 4 * 8 * 64 + threadIdx.x * 8;
+    float v[4][8], A[8], C[8], R[8];
+    for (int w = 0; w < 4; w++)
+        for (int k = 0; k < 8; k++) v[w][k] = p[w * 8 * 64 + k];
+    tprh::quots_rn<8>(v[0], v[1], v[2], v[3], A, C, R);
+    unsigned long long differ = 0;
+    for (int k = 0; k < 8; k++) {
+        differ += !same(A[k], v[0][k] / v[3][k]);
+        differ += !same(C[k], v[1][k] / v[3][k]);
+        differ += !same(R[k], v[2][k] / v[3][k]);
+    }
+    if (differ) atomicAdd(&counts[0], differ);
+    atomicAdd(&counts[1], 24ull);
+}
+
 }  // namespace
+
+// Both return a hipError_t; counts: 2 zeroed words.
+extern "C" int tprh_diag_quot_short_check(int blocks, unsigned first, unsigned stride, unsigned long long* counts,
+                                          void* stream) {
+    hipLaunchKernelGGL(quot_short_check_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, first, stride, counts);
+    return (int)hipGetLastError();
+}
+extern "C" int tprh_diag_quots_check(const float* ops, int blocks, unsigned long long* counts, void* stream) {
+    hipLaunchKernelGGL(quots_check_kernel, dim3(blocks), dim3(64), 0, (hipStream_t)stream, ops, counts);
+    return (int)hipGetLastError();
+}
 
 // counts: 2 zeroed words.  Returns a hipError_t.
 extern "C" int tprh_diag_recip_short_check(unsigned long long* counts, void* stream) {
