@@ -23,6 +23,27 @@ def bits_equal(x, y):
     return bool(np.all(same | (np.isnan(x) & np.isnan(y))))
 
 
+def special_batch(seed, n, s):
+    """One kind of special value per system, spread over every position of a
+    slice."""
+    rng = np.random.default_rng(seed)
+    special = [(0.0, -0.0), (-0.0, -0.0), (np.inf, 1.0), (np.nan, 0.0), (1e-39, -0.0), (3e38, 0.0), (-1e20, 1e30),
+               (1.0, 1.0)]
+    nsys = len(special)
+    a, b, c, d, _ = O.gen_batch(seed + 1, 0, nsys, n, O.GEN_DOMINANT)
+    a, b, c, d = (v.reshape(nsys, n) for v in (a, b, c, d))
+    for k, (off, rhs) in enumerate(special):
+        at = np.unique(np.concatenate([rng.integers(0, n, 12), [0, 1, s - 1, s, n - 2, n - 1]]))
+        b[k] = 1.0
+        for v in (a, c):
+            v[k, at] = np.float32(off)
+        d[k, at[::2]] = np.float32(rhs)
+        if off == 1.0:  # 1 - c a = 0 between neighbours
+            a[k, 1::2], c[k, 0::2] = 1.0, 1.0
+        a[k, 0] = c[k, n - 1] = 0.0
+    return [np.ascontiguousarray(v.ravel(), np.float32) for v in (a, b, c, d)], nsys
+
+
 def gpu(a, b, c, d, n, s, shape=None, **kw):
     da, db, dc, dd = (torch.from_numpy(np.ascontiguousarray(v)).cuda() for v in (a, b, c, d))
     x = torch.full_like(dd, 7.0)
@@ -153,3 +174,21 @@ def test_quotients_of_one_divisor(kind):
                                          ctypes.c_void_p(0)) == 0
     torch.cuda.synchronize()
     assert counts.tolist() == [0, blocks * 64 * 24]
+
+
+TPR_SHAPES = [(2, 16), (4, 16), (4, 64)] + SHAPES
+
+
+@pytest.mark.parametrize("E,L", TPR_SHAPES)
+def test_tpr_shared_branches_bit_identical(E, L):
+    s = E * L
+    n = 2 * s
+    print("exact tpr", E, L, flush=True)
+    (a, b, c, d), nsys = special_batch(76, n, s)
+    x = gpu(a, b, c, d, n, s, (E, L), method="tpr").reshape(nsys, n)
+    with np.errstate(all="ignore"):
+        ref = O.solve_batch("tpr", a, b, c, d, n, s).reshape(nsys, n)
+    for k in range(nsys):
+        assert bits_equal(x[k], ref[k]), k
+    a, b, c, d, _ = O.gen_batch(78, 0, 5, n, O.GEN_WEAK)
+    assert bits_equal(gpu(a, b, c, d, n, s, (E, L), method="tpr"), O.solve_batch("tpr", a, b, c, d, n, s))

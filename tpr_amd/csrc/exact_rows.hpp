@@ -219,6 +219,19 @@ __device__ __forceinline__ void quots_rn(const float (&a)[E], const float (&c)[E
     }
 }
 
+// The two halves of an exact pcr_update (tpr_device.hpp), so that several
+// rows' reciprocals share one range test and branch in between: the
+// denominator and the right-hand side's sum, and the row from the inverse.
+__device__ __forceinline__ void pcr_sums(Eq k, Eq kl, Eq kr, bool hasL, bool hasR, float& den, float& rn) {
+    const float t1 = hasL ? (1.0f - kl.c * k.a) : 1.0f;
+    den = hasR ? (t1 - kr.a * k.c) : t1;
+    rn = hasL ? (k.r - kl.r * k.a) : k.r;
+    rn = settled(hasR ? (rn - kr.r * k.c) : rn);
+}
+__device__ __forceinline__ Eq pcr_row(Eq k, Eq kl, Eq kr, bool hasL, bool hasR, float inv, float rn) {
+    return Eq{hasL ? (-inv * kl.a) * k.a : inv * k.a, hasR ? (-inv * kr.c) * k.c : inv * k.c, inv * rn};
+}
+
 // One level on the blocked layout, u = U < E.
 template <int E, int L, int U>
 __device__ __forceinline__ void exact_level_blocked(float (&Ap)[E], float (&Cp)[E], float (&R)[E], int l) {

@@ -321,6 +321,9 @@ __device__ __forceinline__ void ptpr_stage1_fast16(float (&Ap)[E], float (&Cp)[E
 // original values in Ao/Co/Ro for stage 3 (the reference's bkup of
 // src/tpr.cpp:128-132); odd offsets end with their stage-1 values
 // (src/tpr.cpp:209-213).
+// Exact: the reciprocals of a level's updates share one range test and branch
+// (recips_rn), all sums before them; 4096 systems of N = 1024 18.8 -> 17.7
+// us, 256 of 16384, s = 2048 24.9 -> 22.6.
 // SETTLE: see settled(); not where a lane's 128 registers overflow either way
 // (E = 32 in workgroups of 1024 lanes spills 1756 bytes with it, 596 without).
 template <int E, int L, int MODE, int U, bool SETTLE = true>
@@ -342,28 +345,53 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
             nC[j] = C[j];
             nR[j] = R[j];
         }
+        if constexpr (MODE == kExact && SETTLE) {
+            // updates 2 i and 2 i + 1: the start and the end of block i
+            constexpr int N = 2 * (E / P);
+            Eq kl[N], kr[N];
+            float inv[N], rn[N];
 #pragma unroll
-        for (int j = 0; j < E; j += P) {
-            // block start j
-            {
-                Eq kl = (j >= U) ? Eq{A[j - U], C[j - U], R[j - U]} : left;
-                Eq kr{A[j + U], C[j + U], R[j + U]};
-                bool hasL = (j >= U) || (l > 0);
-                Eq o = pcr_update<MODE, SETTLE>(Eq{A[j], C[j], R[j]}, kl, kr, hasL, true);
-                nA[j] = o.a;
-                nC[j] = o.c;
-                nR[j] = o.r;
+            for (int i = 0; i < N; i++) {
+                const int k = (i / 2) * P + (i & 1) * (P - 1);
+                kl[i] = (k >= U) ? Eq{A[k >= U ? k - U : 0], C[k >= U ? k - U : 0], R[k >= U ? k - U : 0]} : left;
+                kr[i] = (k + U < E) ? Eq{A[k + U < E ? k + U : 0], C[k + U < E ? k + U : 0], R[k + U < E ? k + U : 0]}
+                                    : right;
+                pcr_sums(Eq{A[k], C[k], R[k]}, kl[i], kr[i], k >= U || l > 0, k + U < E || l < L - 1, inv[i], rn[i]);
             }
-            // block end j + P - 1
-            {
-                const int k = j + P - 1;
-                Eq kl{A[k - U], C[k - U], R[k - U]};
-                Eq kr = (k + U < E) ? Eq{A[k + U], C[k + U], R[k + U]} : right;
-                bool hasR = (k + U < E) || (l < L - 1);
-                Eq o = pcr_update<MODE, SETTLE>(Eq{A[k], C[k], R[k]}, kl, kr, true, hasR);
+            recips_rn<N>(inv);
+#pragma unroll
+            for (int i = 0; i < N; i++) {
+                const int k = (i / 2) * P + (i & 1) * (P - 1);
+                const Eq o = pcr_row(Eq{A[k], C[k], R[k]}, kl[i], kr[i], k >= U || l > 0, k + U < E || l < L - 1,
+                                     inv[i], rn[i]);
                 nA[k] = o.a;
                 nC[k] = o.c;
                 nR[k] = o.r;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < E; j += P) {
+                // block start j
+                {
+                    Eq kl = (j >= U) ? Eq{A[j - U], C[j - U], R[j - U]} : left;
+                    Eq kr{A[j + U], C[j + U], R[j + U]};
+                    bool hasL = (j >= U) || (l > 0);
+                    Eq o = pcr_update<MODE, SETTLE>(Eq{A[j], C[j], R[j]}, kl, kr, hasL, true);
+                    nA[j] = o.a;
+                    nC[j] = o.c;
+                    nR[j] = o.r;
+                }
+                // block end j + P - 1
+                {
+                    const int k = j + P - 1;
+                    Eq kl{A[k - U], C[k - U], R[k - U]};
+                    Eq kr = (k + U < E) ? Eq{A[k + U], C[k + U], R[k + U]} : right;
+                    bool hasR = (k + U < E) || (l < L - 1);
+                    Eq o = pcr_update<MODE, SETTLE>(Eq{A[k], C[k], R[k]}, kl, kr, true, hasR);
+                    nA[k] = o.a;
+                    nC[k] = o.c;
+                    nR[k] = o.r;
+                }
             }
         }
 #pragma unroll
@@ -389,8 +417,18 @@ __device__ __forceinline__ void tpr_stage1_level(float (&A)[E], float (&C)[E], f
         Eq el{shift_up<L, D>(e0.a, -1.0f, l), shift_up<L, D>(e0.c, 0.0f, l), shift_up<L, D>(e0.r, 0.0f, l)};
         Eq er{shift_down<L, D>(e0.a, 0.0f, l), shift_down<L, D>(e0.c, -1.0f, l),
               shift_down<L, D>(e0.r, 0.0f, l)};
-        Eq so = pcr_update<MODE, SETTLE>(s0, sl, sr, hasL, hasR);
-        Eq eo = pcr_update<MODE, SETTLE>(e0, el, er, hasL, hasR);
+        Eq so, eo;
+        if constexpr (MODE == kExact && SETTLE) {
+            float inv[2], sn, en;
+            pcr_sums(s0, sl, sr, hasL, hasR, inv[0], sn);
+            pcr_sums(e0, el, er, hasL, hasR, inv[1], en);
+            recips_rn<2>(inv);
+            so = pcr_row(s0, sl, sr, hasL, hasR, inv[0], sn);
+            eo = pcr_row(e0, el, er, hasL, hasR, inv[1], en);
+        } else {
+            so = pcr_update<MODE, SETTLE>(s0, sl, sr, hasL, hasR);
+            eo = pcr_update<MODE, SETTLE>(e0, el, er, hasL, hasR);
+        }
         if (lq == 0) {
             A[0] = so.a;
             C[0] = so.c;
