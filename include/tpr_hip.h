@@ -223,8 +223,8 @@ tprh_status tprh_solve_ex_noalloc(const tprh_solve_desc *desc, void *stream);
  * s = min(n, 256) with its default shape); a system's result depends on its
  * class's entry only, never on the rest of the batch.  Sizes: powers of two
  * from 16 with n / s * L <= 1024.  Creating the plan allocates its device
- * tables; tprh_uneven_solve allocates nothing and is graph-capturable (two
- * kernels: a counter reset and the persistent solver).  A plan holds one work
+ * tables; tprh_uneven_solve allocates nothing and is graph-capturable (one
+ * kernel, for large plans after a counter reset).  A plan holds one work
  * counter, so its solves must not overlap on the device: issue them on one
  * stream (or order them with events); solves that overlap need a plan each. */
 typedef struct tprh_uneven_plan tprh_uneven_plan;

@@ -71,3 +71,23 @@ def test_tiles_every_shape(method, E, L):
     for k, n in enumerate(sizes):
         lo, hi = plan.offset(k), plan.offset(k + 1)
         assert bits_equal(x[lo:hi], O.solve_batch(method, a[lo:hi], b[lo:hi], c[lo:hi], d[lo:hi], n, s)), (k, n)
+
+
+@pytest.mark.parametrize("count", [1, 257, 600, 900])
+def test_items_in_turn_and_by_counter(count):
+    """Plans of 1024-lane items below, between and above one and three items
+    per workgroup (a device of 256 CUs): every answer is written, the same in
+    a second solve."""
+    sizes = [16384] * count + [64]
+    print("items", count, flush=True)
+    plan = UnevenPlan(sizes)
+    a, b, c, d, x, xt = [torch.zeros(plan.equations, device="cuda") for _ in range(6)]
+    plan.generate("dominant", 92, 0, a, b, c, d, xt)
+    for _ in range(2):
+        x.fill_(7.0)
+        plan.solve(a, b, c, d, x)
+        torch.cuda.synchronize()
+        err = (x.double() - xt.double()).view(-1)
+        assert float(err.norm() / xt.double().norm()) < 1e-5
+        # a system left out would be all sevens
+        assert float(err.abs().max()) < 1e-2

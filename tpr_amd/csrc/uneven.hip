@@ -5,10 +5,11 @@
 // per-class table (the autotuner's), and cuts each class into work items of
 // as many systems as one workgroup holds: 256 lanes where all of the plan's
 // systems fit them, one workgroup per item, else 1024 lanes in a persistent
-// kernel.  That one keeps one workgroup per resident slot; where there are
-// more items, each workgroup takes the next from an atomic counter (items are
-// ordered largest systems first) and asks for its next ticket as it starts an
-// item, so the counter's latency hides under the item.  Every system's result
+// kernel.  That one keeps one workgroup per resident slot.  Up to kSweepRounds
+// items each it takes them in turn; beyond, each workgroup takes the next from
+// an atomic counter (items are ordered largest systems first) and asks for its
+// next ticket as it starts an item, so the counter's latency hides under the
+// item.  Every system's result
 // depends only on its own size class's (s, E, L), never on the batch around
 // it.
 #include <hip/hip_runtime.h>
@@ -51,7 +52,7 @@ __device__ __forceinline__ void run_shape(const UnevenTask& tk, const int* __res
 
 __global__ void zero_counter_kernel(int* counter) { *counter = 0; }
 
-// counter NULL: a workgroup per item.
+// counter NULL: workgroup k takes the items k, k + grid, ...
 template <int METHOD, int MODE, bool HAS_B>
 __global__ __launch_bounds__(kSlotBig) void uneven_kernel(const UnevenTask* __restrict__ tasks, int ntasks,
                                                           int* __restrict__ counter, const int* __restrict__ sys_list,
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(kSlotBig) void uneven_kernel(const UnevenTask* __re
         // the counter is device-coherent, its answer takes microseconds
         // behind the memory traffic, and this item's loads now cover that
         // wait (a workgroup holds at most two tickets; items are independent)
-        int nxt = ntasks;
+        int nxt = it + (int)gridDim.x;
         if (threadIdx.x == 0 && counter) nxt = next_ticket(counter);
         run_shape<METHOD, MODE, HAS_B, kSlotBig>(tasks[it], sys_list, offsets, a, b, c, d, x, lds);
         __syncthreads();  // the item's LDS rows are read before the next item writes them;
@@ -96,6 +97,12 @@ __global__ __launch_bounds__(kSlotTile, 4) void uneven_tile_kernel(const UnevenT
 
 namespace {
 
+// Items per workgroup up to which they are taken in turn: the counter's clear
+// is a launch of 5 us, and what the counter balances grows with the items.
+// Systems of 256 .. 16384, counter -> in turn: 1300 (1.5 items) 38.9 -> 34.1
+// us, 2500 (2.8) 67.2 -> 66.1, 4000 (4.4) 94.4 -> 103, 20000 (22) 385 -> 404.
+constexpr int kSweepRounds = 3;
+
 template <int METHOD, int MODE, bool HAS_B>
 hipError_t allow_big_lds() {
     static std::atomic<unsigned long long> set{0};
@@ -109,7 +116,7 @@ hipError_t launch_uneven_t(const UnevenLaunch& p, hipStream_t stream) {
     if (p.block == kSlotBig) {
         hipError_t e = allow_big_lds<METHOD, MODE, HAS_B>();
         if (e != hipSuccess) return e;
-        int* counter = p.ntasks > p.grid ? p.counter : nullptr;
+        int* counter = p.ntasks > kSweepRounds * (long long)p.grid ? p.counter : nullptr;
         if (counter) hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
         hipLaunchKernelGGL((uneven_kernel<METHOD, MODE, HAS_B>), dim3(p.grid), dim3(kSlotBig),
                            slot_big_lds(METHOD, MODE), stream, p.tasks, p.ntasks, counter, p.sys_list, p.offsets, p.a,
