@@ -318,7 +318,10 @@ tprh_status tprh_server_matrix_release(tprh_server *srv, long long matrix);
  * the answers go (nrhs * n floats, host or device) when the request
  * completes, or NULL to keep them in the arena until
  * tprh_server_request_release (tprh_server_request_info gives the device
- * address).  TPRH_ERROR_BUDGET: the request needs more than the whole arena.
+ * address).  A 16-byte aligned x in this device's memory is written by the
+ * solve itself, so parts of it may change before the request completes, and
+ * what it holds after a failure is unspecified.  TPRH_ERROR_BUDGET: the
+ * request needs more than the whole arena.
  * Host d and x should be pinned (hipHostMalloc) or device memory: both are
  * copied by hipMemcpyAsync on the batch's stream (d before its kernels, x
  * after them), and a copy from or to pageable host memory may make the

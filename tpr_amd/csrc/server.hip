@@ -339,8 +339,8 @@ struct Staged {
 // entries, generation jobs, the serve kernel's zeroed work counter) is
 // packed into the slot's pinned staging buffer and copied with one
 // transfer; then, on the slot's stream: caller right-hand sides are copied
-// in (those in this device's memory by one kernel), synthetic ones and the coefficients of matrices first used here are
-// generated (one launch, then the gen_done event that batches on other
+// in (those in this device's memory by one kernel), synthetic ones and the
+// coefficients of matrices first used here are generated (one launch, then the gen_done event that batches on other
 // slots using those matrices wait for), the serve kernel runs for every
 // class within a workgroup, one split launch set per larger class, and the
 // answers the caller asked for are copied out -- those for 16-byte aligned

@@ -7,9 +7,9 @@
 // barriers and limits n to s^2 (src/ptpr.cu:543,581,655).  Here a batch is
 // solved in rounds of `chunk` systems, each round in one of four forms:
 //
-// Fused (split_fused.hpp), the library's form for fast PTPR and TPR at s >= 256 (and
-// what split_form 2 asks for there): one pass over tiles that exchange six
-// numbers each, 63.5 us for 256 x N=65536.
+// Fused (split_fused.hpp), the library's form for fast PTPR and TPR at
+// s >= 256 (and what split_form 2 asks for there): one pass over tiles that
+// exchange six numbers each, 63.5 us for 256 x N=65536.
 //
 // Two passes (split_kernels.hpp), the library's form for everything else:
 //   K1 rows_kernel   : every lane group reduces its slices and writes two
@@ -29,9 +29,8 @@
 // vs src/ptpr.cpp:140-182), so in exact arithmetic K1 runs the O(S) tree for
 // both methods and its rows are bit-identical to the full PCR's.  In fast
 // arithmetic, PTPR on 16-lane slices runs the two-level stage 1 in K1 and K3
-// (as the one-workgroup path does), which also keeps both kernels at 72-78
-// VGPRs, 6-7 waves per SIMD: on MI355X the 256 x 65536 batch takes 41 + 6 +
-// 50 us this way against 42 + 6 + 58 us with the register PCR in K3.
+// (as the one-workgroup path does): on MI355X the 256 x 65536 batch takes 46
+// + 6 + 47 us this way.
 //
 // One pass (persistent_split_kernel), on request (split_form 2): each block
 // keeps its slices in registers from the load to the store and waits for
@@ -48,9 +47,9 @@
 // the reloads it saves, which the last-level cache serves only about 1.4x
 // faster than HBM on this part.
 //
-// Exact answers are the same bits in every
-// form (the same operations in the same order); fast answers agree within
-// rounding (the forms differ in where stage 1's end rows come from).
+// Exact answers are the same bits in every form (the same operations in the
+// same order); fast answers agree within rounding (the forms differ in where
+// stage 1's end rows come from).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -63,8 +63,9 @@ template <int E, int MODE>
 constexpr int kExactWaves = MODE == kExact && E <= 16 ? 4 : 1;
 
 // K1 and K3 load (and K3 stores) their slices as 1 KB runs per instruction
-// through LDS (staged_io.hpp) where the shape stages: a wavefront holds 64 / L whole slices of one system (m L > 1024), one
-// contiguous run starting at `run`.  256-lane workgroups: four wavefronts.
+// through LDS (staged_io.hpp) where the shape stages: a wavefront holds 64 / L
+// whole slices of one system (m L > 1024), one contiguous run starting at
+// `run`.  256-lane workgroups: four wavefronts.
 // K3 stores x non-temporally (256 x N=65536: 0.0951-0.0955 against
 // 0.0965-0.0968 ms with cached stores).
 template <int E, typename CT>
