@@ -84,19 +84,6 @@ struct RawPart {
     float a[E], b[E], c[E], d[E];
 };
 
-// Branch-free: a lane of a system past the end of the batch loads the same
-// lane of system 0 (always present) and never stores, so the loads stay in
-// one basic block and the compiler keeps them where they are issued.
-template <int E>
-__device__ __forceinline__ void load_raw(const float* __restrict__ a, const float* __restrict__ b,
-                                         const float* __restrict__ c, const float* __restrict__ d, size_t off,
-                                         RawPart<E>& p) {
-    load_e<E>(a + off, p.a);
-    load_e<E>(c + off, p.c);
-    load_e<E>(d + off, p.d);
-    if (b != nullptr) load_e<E>(b + off, p.b);
-}
-
 // E consecutive fp16 values, widened to fp32 (exact).
 template <int E>
 __device__ __forceinline__ void load_e(const _Float16* __restrict__ p, float (&v)[E]) {
