@@ -155,6 +155,19 @@ def test_one_pass_sweeps_that_are_not_all_there(n, nsys, stride, parts, spin, re
     assert np.array_equal(bits(x), bits(ref))
 
 
+@pytest.mark.parametrize("refine", [False, True])
+@pytest.mark.parametrize("n,nsys,stride,parts,spin", [
+    (1 << 19, 1, 128, [(0, 64), (64, 64)], 0),    # whole groups of tiles absent, one tile per workgroup
+    (1 << 19, 1, 128, [(32, 96), (0, 32)], 1),
+    (1 << 17, 2, 64, [(0, 16), (16, 48)], 0),     # of one system one group, of the other none
+    (1 << 19, 2, 256, [(112, 16), (128, 128), (0, 112)], 2),
+])
+def test_one_pass_sweeps_without_whole_groups(n, nsys, stride, parts, spin, refine):
+    """Groups none of whose workgroups is there: each launch publishes their
+    tiles and their groups and finishes its own."""
+    test_one_pass_sweeps_that_are_not_all_there(n, nsys, stride, parts, spin, refine)
+
+
 def test_one_pass_in_a_graph_and_on_streams():
     """Replays of a captured solve, with eager work between them, and two
     solves overlapping on two streams: the eager answers' bits."""

@@ -1,0 +1,90 @@
+// fused_walk.hpp -- what a workgroup of the one-pass form (split_fused.hpp)
+// does next: its own tiles first, then those it had to put aside, and in
+// between the tiles that others have not published.  Host and device code
+// alike, so that a CPU test can run the same decisions for many sets of
+// workgroups of which only some are there.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace tprh {
+
+constexpr int kFusedGroup = 16;  // tiles per group (one DPP row)
+
+// A workgroup's next task: a tile of its own, one of its own taken up again,
+// or one of another workgroup published on its behalf.
+enum FusedKind { kFusedOwn = 0, kFusedAgain = 1, kFusedHelp = 2 };
+
+// One of the set bits of `missing`: the first from bit `from` on, or else the
+// first of all, so that workgroups which wait for the same blocks start on
+// different ones.
+__host__ __device__ inline int fused_pick(unsigned long long missing, int from) {
+    const unsigned long long above = missing >> from << from;
+    return __builtin_ctzll(above ? above : missing);
+}
+
+// Systems of more than 16 tiles: -1 once every group's words are there for
+// tile ti, else a tile (in the system) that is missing.  x.tiles(g, limit)
+// and x.groups(limit) poll up to `limit` more times for the 16 tiles of group
+// g and for the groups, and return which are missing; x.publish(g) publishes
+// group g from the tiles just read.  A tile waiting for the first time
+// (`first`) only asks; afterwards a group whose tiles are all there, but
+// whose first tile's workgroup is not, is published here, so that what is
+// returned is always a tile not yet published when it was looked at.
+template <typename X>
+__host__ __device__ __forceinline__ int fused_look(X& x, bool first, int ti, int limit) {
+    const int g = ti / kFusedGroup;
+    unsigned long long m = x.tiles(g, limit);
+    if (m != 0) return g * kFusedGroup + fused_pick(m, ti % kFusedGroup);
+    x.publish(g);
+    for (;;) {  // ends: each turn but the last publishes a missing group
+        m = x.groups(limit);
+        if (m == 0) return -1;
+        const int other = fused_pick(m, g);
+        if (first) return other * kFusedGroup;
+        m = x.tiles(other, 0);
+        if (m != 0) return other * kFusedGroup + fused_pick(m, ti % kFusedGroup);
+        x.publish(other);
+        limit = 0;
+    }
+}
+
+struct FusedTask {
+    int tile;  // -1: the workgroup is done
+    int kind;
+};
+
+// The lists of one workgroup, kept by its thread 0: tiles of its own whose
+// system was not all there in time (linked through the workspace), and those
+// taken up again in vain.
+struct FusedWalk {
+    int head = -1, again = -1;
+    int tries = 0;  // tasks beyond its own tiles
+
+    // After task (tile, kind): ok, the system was all there (and an own
+    // tile's x is stored); missing, a tile of it that was not.  own: the
+    // workgroup's next own tile, -1 when it has none left.  A tile taken up
+    // again in vain is followed by help with one missing tile after the
+    // other until its system is all there.
+    template <typename Link>
+    __host__ __device__ __forceinline__ FusedTask next(int tile, int kind, bool ok, int missing, int own, int limit,
+                                                       Link&& link) {
+        if (!ok && kind != kFusedHelp) {
+            int& to = kind == kFusedOwn ? head : again;
+            link(tile) = to;
+            to = tile;
+        }
+        if (own >= 0) return {own, kFusedOwn};
+        if (tries >= limit) return {-1, kFusedAgain};
+        tries++;
+        if (!ok && kind != kFusedOwn) return {missing, kFusedHelp};
+        if (head < 0) {
+            head = again;
+            again = -1;
+        }
+        const int t = head;
+        if (t >= 0) head = link(t);
+        return {t, kFusedAgain};
+    }
+};
+
+}  // namespace tprh

@@ -39,35 +39,31 @@
 // form, everything else alike (256 x N=65536, one
 // buffer set: 100 us two passes, 58 us).
 //
-// The solve ends whichever workgroups are resident.  Workgroup k of a grid of
-// G takes tiles k, k + G, ...; it publishes a tile before it waits, and waits
-// only `spin` polls: then it puts the tile on a list (linked through the
-// workspace) and goes on with its next one.  Its own tiles done, it takes the
-// listed ones up again (loading them again); where one still misses a tile,
-// that tile's workgroup may not have started, and it computes and publishes
-// the missing tile on that workgroup's behalf (the same words), so each
-// workgroup can finish with no other's help.  With a grid that the device
-// holds at once, as launched here, on an otherwise idle device, no tile is
-// ever listed.
+// The solve ends whichever workgroups are resident (fused_walk.hpp).
+// Workgroup k of a grid of G takes tiles k, k + G, ...; it publishes a tile
+// before it waits, and waits only `spin` polls: then it puts the tile on a
+// list (linked through the workspace) and goes on with its next one.  Its own
+// tiles done, it takes the listed ones up again (loading them again); where
+// one still misses a tile, that tile's workgroup may not have started, and it
+// computes and publishes the system's missing tiles, one after the other, on
+// their workgroups' behalf (the same words), so each workgroup can finish
+// with no other's help.  With a grid that the device holds at once, as
+// launched here, on an otherwise idle device, no tile is ever listed.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 
+#include "fused_walk.hpp"
 #include "split_kernels.hpp"
 
 namespace tprh {
 
 constexpr int kFusedTile = 4096;               // equations per workgroup
 constexpr int kFusedThreads = 256;
-constexpr int kFusedGroup = 16;                // tiles per group (one DPP row)
 constexpr unsigned kFusedEmpty = 0xffffffffu;  // a word not yet published
 constexpr int kFusedSpin = 64;                 // polls (about a microsecond each) before a tile is listed
 constexpr int kFusedTries = 1 << 14;           // tasks of one workgroup beyond its own tiles, in all
-
-// A workgroup's next task: a tile of its own, one of its own taken up again,
-// or one of another workgroup published on its behalf.
-enum FusedKind { kFusedOwn = 0, kFusedAgain = 1, kFusedHelp = 2 };
 
 // What the workgroups of one system exchange, in its boundary buffer (Rows)
 // of bps tiles.  For block t (a tile; behind them a group of 16 tiles), its
@@ -305,6 +301,31 @@ struct RowState<1, E> {  // TPR: the tree (src/tpr.cpp:123-230, :277-308)
     }
 };
 
+// What a wavefront reads and publishes of a system of groups (fused_look).
+struct GroupWords {
+    const FusedWords fw;
+    const int lane, own;  // own: the tile's group
+    BlockEnds e;          // of the blocks last read, one per lane; past the last one zero equations
+    Chain16 chain;        // of the own group, once published
+
+    __device__ __forceinline__ unsigned long long tiles(int g, int limit) {
+        const int t = g * kFusedGroup + (lane & 15);
+        e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        return wait_ends(fw.ends4(t), fw.ends2(t), lane < kFusedGroup, limit, e);
+    }
+    __device__ __forceinline__ unsigned long long groups(int limit) {
+        e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        return wait_ends(fw.group4(lane), fw.group2(lane), lane < fw.groups(), limit, e);
+    }
+    __device__ __forceinline__ void publish(int g) {
+        Chain16 c;
+        c.reduce(e, lane & 15);
+        const BlockEnds ge = c.ends(0);
+        if (lane == 0) publish_ends(fw.group4(g), fw.group2(g), ge);
+        if (g == own) chain = c;
+    }
+};
+
 // WIDE: more than 16 tiles per system (up to 1024): the exchange goes through
 // groups of 16 tiles -- the group's first tile reduces it, exchanges its ends
 // with the other groups', and hands every tile of the group the x on its
@@ -334,9 +355,8 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
     // whole chip to 47 tiles a microsecond: 86 us for 256 x N=65536)
     int own = first + (int)blockIdx.x;
     int tile = own, kind = kFusedOwn;
-    // thread 0: the workgroup's listed tiles, those taken up again in vain,
-    // a tile to help with, and the tasks taken beyond its own tiles
-    int head = -1, again = -1, missing = -1, tries = 0;
+    FusedWalk walk;    // thread 0's
+    int missing = -1;  // a tile to help with
     while (tile >= 0 && tile < total) {  // uniform
         const int q = tile >> lg_bps;
         const int ti = tile & (bps - 1);
@@ -410,48 +430,38 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             }
             BlockEnds e{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             float before = 0.0f, after = 0.0f;
-            unsigned long long m;  // lanes whose block is missing
+            bool there;  // every block that this tile waits for
             const int limit = kind == kFusedHelp ? 0 : spin;
             if constexpr (!WIDE) {
-                m = wait_ends(fw.ends4(lane), fw.ends2(lane), lane < bps, limit, e);
-                if (m == 0) solve_blocks<false>(e, bps, ti, lane, before, after);
-                else missing = tile - ti + __builtin_ctzll(m);
+                const unsigned long long m = wait_ends(fw.ends4(lane), fw.ends2(lane), lane < bps, limit, e);
+                there = m == 0;
+                if (there) solve_blocks<false>(e, bps, ti, lane, before, after);
+                else missing = tile - ti + fused_pick(m, ti);
+            } else if (ti % kFusedGroup != 0 && kind == kFusedOwn) {
+                there = wait_pair(fw.result(ti), lane, limit, before, after) == 0;
             } else {
-                const int g = ti / kFusedGroup, ng = fw.groups();
                 // the group's first tile reduces the group, solves the system
                 // of the groups and hands every tile of the group its sides
                 // (a tile taken up again does so by itself)
-                if (ti % kFusedGroup != 0 && kind == kFusedOwn) {
-                    m = wait_pair(fw.result(ti), lane, limit, before, after);
+                const int g = ti / kFusedGroup;
+                GroupWords gw{fw, lane, g};
+                const int lost = fused_look(gw, kind == kFusedOwn, ti, limit);
+                there = lost < 0;
+                if (there) {
+                    float ob, oa, xb, xe, xa;
+                    solve_blocks<true>(gw.e, fw.groups(), g, lane, ob, oa);
+                    gw.chain.solve(ob, oa, l, xb, xe, xa);
+                    if (lane < kFusedGroup) publish_pair(fw.result(g * kFusedGroup + l), xb, xa);
+                    before = __shfl(xb, ti % kFusedGroup, 64);
+                    after = __shfl(xa, ti % kFusedGroup, 64);
                 } else {
-                    const int t = g * kFusedGroup + l;
-                    m = wait_ends(fw.ends4(t), fw.ends2(t), lane < kFusedGroup, limit, e);
-                    if (m != 0) {
-                        missing = tile - ti + g * kFusedGroup + __builtin_ctzll(m);
-                    } else {
-                        Chain16 cg;
-                        cg.reduce(e, l);
-                        const BlockEnds ge = cg.ends(0);
-                        if (threadIdx.x == 0) publish_ends(fw.group4(g), fw.group2(g), ge);
-                        e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-                        m = wait_ends(fw.group4(lane), fw.group2(lane), lane < ng, limit, e);
-                        if (m != 0) {
-                            missing = tile - ti + __builtin_ctzll(m) * kFusedGroup + tries % kFusedGroup;
-                        } else {
-                            float ob, oa, xb, xe, xa;
-                            solve_blocks<true>(e, ng, g, lane, ob, oa);
-                            cg.solve(ob, oa, l, xb, xe, xa);
-                            if (lane < kFusedGroup) publish_pair(fw.result(t), xb, xa);
-                            before = __shfl(xb, ti % kFusedGroup, 64);
-                            after = __shfl(xa, ti % kFusedGroup, 64);
-                        }
-                    }
+                    missing = tile - ti + lost;
                 }
             }
             if (threadIdx.x == 0) {
                 s_side[0] = before;
                 s_side[1] = after;
-                s_ok = m == 0 ? 1 : 0;
+                s_ok = there ? 1 : 0;
             }
         }
         __syncthreads();
@@ -476,33 +486,12 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         }
         // a tile to list, or no tile of its own left
         if (threadIdx.x == 0) {
-            if (!ok && kind != kFusedHelp) {
-                int& to = kind == kFusedOwn ? head : again;
-                *fw.link(ti) = to;
-                to = tile;
-            }
-            int t = -1, k = kFusedAgain;
-            if (own + stride < total) {
-                t = own + stride;
-                k = kFusedOwn;
-            } else if (tries < kFusedTries) {
-                if (!ok && kind == kFusedAgain) {
-                    t = missing;
-                    k = kFusedHelp;
-                } else {
-                    if (head < 0) {
-                        head = again;
-                        again = -1;
-                    }
-                    if (head >= 0) {
-                        t = head;
-                        head = *FusedWords{loc.Rows(t >> lg_bps), bps}.link(t & (bps - 1));
-                    }
-                }
-                tries++;
-            }
-            s_tile = t;
-            s_kind = k;
+            const FusedTask t = walk.next(tile, kind, ok, missing, own + stride < total ? own + stride : -1, kFusedTries,
+                                          [&](int k) -> int& {
+                                              return *FusedWords{loc.Rows(k >> lg_bps), bps}.link(k & (bps - 1));
+                                          });
+            s_tile = t.tile;
+            s_kind = t.kind;
         }
         __syncthreads();
         tile = __builtin_amdgcn_readfirstlane(s_tile);
