@@ -72,6 +72,7 @@ struct Group {  // a workgroup
         }
         if (!ok && kind == kFusedOwn && patient) return;
         step = 0;
+        if (!ok && kind == kFusedAgain && walk.lost(limit)) ok = true;  // x becomes NaN
         if (ok && kind != kFusedHelp) s.x[tile] = 1;
         const int next = own + stride < s.total ? own + stride : -1;
         const FusedTask t = walk.next(tile, kind, ok, missing, next, limit, [&](int k) -> int& { return s.link[k]; });
@@ -161,3 +162,50 @@ int main() {
 }
 ''' % ", ".join("%du" % k for k in seeds))
     assert int(out) == len(seeds) * 6 * 2 * 5 * 9
+
+
+def test_the_bound_on_tasks_is_never_reached(tmp_path):
+    """Many systems per workgroup and few workgroups there: none needs more
+    tasks than the launch allows it."""
+    out = run(tmp_path, r'''
+int main() {
+    int n = 0;
+    for (int bps : {8, 64, 1024})
+        for (int nsys : {1, 16, 64})
+            for (int stride : {bps, 1024}) {
+                const int total = bps * nsys;
+                if (stride > total) continue;
+                const int limit = fused_task_limit(total, stride, bps);
+                for (const auto& v : {range(0, 1), range(stride - 1, stride), range(0, 16), range(0, stride, 97)}) {
+                    if ((int)v.size() > stride || v.back() >= stride) continue;
+                    const int most = solve(bps, nsys, stride, v, limit, 0);
+                    if (most < 0 || most > limit) {
+                        printf("%d tiles, %d systems, stride %d, %d there: %d of %d tasks\n", bps, nsys, stride,
+                               (int)v.size(), most, limit);
+                        return 1;
+                    }
+                    n++;
+                }
+            }
+    printf("%d", n);
+}
+''')
+    assert int(out) >= 40
+
+
+def test_a_workgroup_out_of_tasks_leaves_no_tile_as_it_was(tmp_path):
+    """With too low a bound (which words changed by another launch could make
+    it): every own tile ends solved or marked as lost."""
+    run(tmp_path, r'''
+int main() {
+    for (int more : {0, 1, 2, 7, 40})
+        for (int bps : {8, 16, 64})
+            for (int stride : {bps, 5, 3 * bps}) {
+                const int limit = (3 * bps + stride - 1) / stride + more;  // own tiles and a few
+                if (solve(bps, 3, stride, range(0, 2), limit, 0) < 0) {
+                    printf("limit %d: %d tiles, stride %d\n", limit, bps, stride);
+                    return 1;
+                }
+            }
+}
+''')

@@ -168,6 +168,31 @@ def test_one_pass_sweeps_without_whole_groups(n, nsys, stride, parts, spin, refi
     test_one_pass_sweeps_that_are_not_all_there(n, nsys, stride, parts, spin, refine)
 
 
+@pytest.mark.parametrize("refine", [False, True])
+@pytest.mark.parametrize("n,nsys,stride,first,blocks", [(65536, 2, 16, 0, 3), (1 << 17, 1, 32, 16, 2)])
+def test_one_pass_tile_given_up_is_nan(n, nsys, stride, first, blocks, refine):
+    """A workgroup that has used up its tasks answers its tiles with NaN; the
+    tiles of those that never came keep what x held."""
+    say("given up", n, nsys, stride, first, blocks, refine)
+    L = _diag()
+    L.tprh_diag_split_fused_bounded.restype = ctypes.c_int
+    a, b, c, d, _ = O.gen_batch(66, 0, nsys, n)
+    da, db, dc, dd = dev(a), dev(b), dev(c), dev(d)
+    x = torch.full((nsys * n,), 2.5, device="cuda")
+    ws = torch.empty(B.workspace_bytes(B.make_desc(da, db, dc, dd, x, n, 256)), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    p = ctypes.c_void_p
+    st = L.tprh_diag_split_fused_bounded(*(p(v.data_ptr()) for v in (da, db, dc, dd, x)), n, nsys, int(refine),
+                                         p(ws.data_ptr()), 1, first, blocks, stride, 0, nsys, p(0))
+    assert st == 0
+    torch.cuda.synchronize()
+    tiles = x.view(-1, 4096)
+    there = [k for k in range(nsys * n // 4096) if first <= k % stride < first + blocks]
+    nan = torch.isnan(tiles).all(1).cpu().numpy()
+    assert sorted(np.flatnonzero(nan)) == there
+    assert bool((tiles[~torch.from_numpy(nan).cuda()] == 2.5).all())
+
+
 def test_one_pass_in_a_graph_and_on_streams():
     """Replays of a captured solve, with eager work between them, and two
     solves overlapping on two streams: the eager answers' bits."""

@@ -48,6 +48,15 @@ __host__ __device__ __forceinline__ int fused_look(X& x, bool first, int ti, int
     }
 }
 
+// Tasks that a workgroup can need beyond its own tiles, of which it has at
+// most total / stride, rounded up: each is taken up again, all other tiles of
+// its system are published, it is taken up once more; at the end there is no
+// tile left.  Only words or lists that something else changes (two
+// overlapping solves in one workspace) can make it need more.
+__host__ __device__ inline int fused_task_limit(int total, int stride, int bps) {
+    return ((total + stride - 1) / stride) * (bps + 2) + 1;
+}
+
 struct FusedTask {
     int tile;  // -1: the workgroup is done
     int kind;
@@ -59,6 +68,11 @@ struct FusedTask {
 struct FusedWalk {
     int head = -1, again = -1;
     int tries = 0;  // tasks beyond its own tiles
+
+    // Past `limit` tasks (fused_task_limit) no tile is waited for or helped
+    // with any more: the caller answers one taken up again in vain with NaN,
+    // as if all were there.  limit: no less than the workgroup's own tiles.
+    __host__ __device__ __forceinline__ bool lost(int limit) const { return tries > limit; }
 
     // After task (tile, kind): ok, the system was all there (and an own
     // tile's x is stored); missing, a tile of it that was not.  own: the
@@ -74,9 +88,9 @@ struct FusedWalk {
             to = tile;
         }
         if (own >= 0) return {own, kFusedOwn};
-        if (tries >= limit) return {-1, kFusedAgain};
+        if (tries > 2 * limit + 2) return {-1, kFusedAgain};  // a list without an end
         tries++;
-        if (!ok && kind != kFusedOwn) return {missing, kFusedHelp};
+        if (!ok && kind != kFusedOwn && tries <= limit) return {missing, kFusedHelp};
         if (head < 0) {
             head = again;
             again = -1;

@@ -48,7 +48,10 @@
 // computes and publishes the system's missing tiles, one after the other, on
 // their workgroups' behalf (the same words), so each workgroup can finish
 // with no other's help.  With a grid that the device holds at once, as
-// launched here, on an otherwise idle device, no tile is ever listed.
+// launched here, on an otherwise idle device, no tile is ever listed.  The
+// tasks that a workgroup can need have a bound (fused_task_limit), which only
+// solves that overlap in one workspace, against its rule, could reach: a tile
+// is then answered with NaN.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -63,7 +66,6 @@ constexpr int kFusedTile = 4096;               // equations per workgroup
 constexpr int kFusedThreads = 256;
 constexpr unsigned kFusedEmpty = 0xffffffffu;  // a word not yet published
 constexpr int kFusedSpin = 64;                 // polls (about a microsecond each) before a tile is listed
-constexpr int kFusedTries = 1 << 14;           // tasks of one workgroup beyond its own tiles, in all
 
 // What the workgroups of one system exchange, in its boundary buffer (Rows)
 // of bps tiles.  For block t (a tile; behind them a group of 16 tiles), its
@@ -336,7 +338,7 @@ struct GroupWords {
 // all of up to 64 tiles' words, 64 systems of 256 Ki 73 us, this way 59.
 template <int METHOD, bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
 __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_kernel(Loc loc, int nsys, int lg_bps, int first,
-                                                                                    int stride, int spin) {
+                                                                                    int stride, int spin, int tasks) {
     constexpr int E = 16;
     __shared__ __align__(16) float stage_lds[stage_words<E>(kFusedThreads)];
     __shared__ float s_ends[6][16];  // E_st and E_ed of the tile's rows
@@ -459,9 +461,10 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
                 }
             }
             if (threadIdx.x == 0) {
-                s_side[0] = before;
-                s_side[1] = after;
-                s_ok = there ? 1 : 0;
+                const bool lost = !there && kind == kFusedAgain && walk.lost(tasks);  // its x: NaN
+                s_side[0] = lost ? __builtin_nanf("") : before;
+                s_side[1] = lost ? __builtin_nanf("") : after;
+                s_ok = there || lost ? 1 : 0;
             }
         }
         __syncthreads();
@@ -486,7 +489,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         }
         // a tile to list, or no tile of its own left
         if (threadIdx.x == 0) {
-            const FusedTask t = walk.next(tile, kind, ok, missing, own + stride < total ? own + stride : -1, kFusedTries,
+            const FusedTask t = walk.next(tile, kind, ok, missing, own + stride < total ? own + stride : -1, tasks,
                                           [&](int k) -> int& {
                                               return *FusedWords{loc.Rows(k >> lg_bps), bps}.link(k & (bps - 1));
                                           });
@@ -535,7 +538,8 @@ hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, b
     const long long pieces = (long long)nsys * fused_clear_pieces(1 << lg_bps);
     hipLaunchKernelGGL((clear_fused_kernel<Loc>), dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, loc,
                        nsys, 1 << lg_bps);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(kFusedThreads), 0, stream, loc, nsys, lg_bps, 0, grid, kFusedSpin);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kFusedThreads), 0, stream, loc, nsys, lg_bps, 0, grid, kFusedSpin,
+                       fused_task_limit(tiles, grid, 1 << lg_bps));
     return hipGetLastError();
 }
 

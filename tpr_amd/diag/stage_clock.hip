@@ -158,11 +158,13 @@ extern "C" int tprh_diag_ptpr_stage_clock(const float* a, const float* b, const 
 // first .. first + blocks - 1 of `stride`, each giving up a wait after `spin`
 // polls: a sweep whose workgroups are not all there, which lists its tiles
 // and publishes the absent ones'.  clear: empty the published words first
-// (the first of several launches that make up one solve).  workspace as
+// (the first of several launches that make up one solve).  tasks: the bound
+// on a workgroup's tasks beyond its own tiles, 0 for the library's, else no
+// less than those (tprh_diag_split_fused: the library's).  workspace as
 // tprh_workspace_bytes gives for s = 256, chunk = nsys.  Returns a hipError_t.
-extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float* c, const float* d, float* x, int n,
-                                     int nsys, int refine, void* workspace, int clear, int first, int blocks,
-                                     int stride, int spin, void* stream) {
+extern "C" int tprh_diag_split_fused_bounded(const float* a, const float* b, const float* c, const float* d, float* x,
+                                             int n, int nsys, int refine, void* workspace, int clear, int first,
+                                             int blocks, int stride, int spin, int tasks, void* stream) {
     using namespace tprh;
     const int m = n / 256;
     if (n % kFusedTile || (n & (n - 1)) || m > kSplitMaxM || nsys < 1 || first < 0 || blocks < 1 ||
@@ -185,8 +187,15 @@ extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float
                                 : fused_split_kernel<0, true, float, true, false, BatchLoc<float>>)
                         : (wide ? fused_split_kernel<0, true, float, false, true, BatchLoc<float>>
                                 : fused_split_kernel<0, true, float, false, false, BatchLoc<float>>);
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), 0, st, loc, nsys, lg, first, stride, spin);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kFusedThreads), 0, st, loc, nsys, lg, first, stride, spin,
+                       tasks ? tasks : fused_task_limit(nsys << lg, stride, 1 << lg));
     return (int)hipGetLastError();
+}
+extern "C" int tprh_diag_split_fused(const float* a, const float* b, const float* c, const float* d, float* x, int n,
+                                     int nsys, int refine, void* workspace, int clear, int first, int blocks,
+                                     int stride, int spin, void* stream) {
+    return tprh_diag_split_fused_bounded(a, b, c, d, x, n, nsys, refine, workspace, clear, first, blocks, stride, spin,
+                                         0, stream);
 }
 
 // The pipelined split solve of nsys fast-PTPR systems of n equations, s = 256
