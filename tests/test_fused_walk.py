@@ -20,6 +20,7 @@ struct Solve {
     int bps, nsys, total;
     std::vector<char> tile, group, result, x;  // published words, stored answers
     std::vector<int> link;
+    bool spoiled = false;  // published from inputs that an answer had taken the place of (x stored over d)
     int ngroups() const { return bps / kFusedGroup; }
     Solve(int b, int s) : bps(b), nsys(s), total(b * s), tile(total), group(total), result(total), x(total), link(total) {}
 };
@@ -43,16 +44,23 @@ struct Words {
 
 struct Group {  // a workgroup
     int own, stride, tile, kind = kFusedOwn, missing = -1, step = 0;
+    bool fresh = false, seen = false;  // what was loaded were inputs; the tile was published after that
     FusedWalk walk;
     Group(int first, int st) : own(first), stride(st), tile(first) {}
     bool done(const Solve& s) const { return tile < 0 || tile >= s.total; }
 
-    // One step: publishing the tile, or looking and going on.  patient: an
-    // own tile's first wait goes on rather than give up.
+    // One step: loading the tile, asking whether it is published, publishing
+    // it, or looking and going on.  patient: an own tile's first wait goes on
+    // rather than give up.
     void run(Solve& s, int limit, bool patient) {
-        if (step == 0) {
-            if (kind != kFusedAgain) s.tile[tile] = 1;
-            step = 1;
+        if (step < 3) {
+            if (step == 0) fresh = !s.x[tile];
+            if (step == 1) seen = s.tile[tile];
+            if (step == 2 && fused_publishes(kind, seen)) {
+                s.tile[tile] = 1;
+                if (!fresh) s.spoiled = true;
+            }
+            step++;
             return;
         }
         const int ti = tile % s.bps, base = tile - ti;
@@ -84,7 +92,8 @@ struct Group {  // a workgroup
 
 // The workgroups `there` of `stride`, and no other: in turn, or with their
 // steps mixed (seed > 0).  Returns the most tasks one took beyond its own
-// tiles, or -1 if a tile of theirs is left.
+// tiles, or -1 if a tile of theirs is left or was published from what x had
+// been stored over.
 int solve(int bps, int nsys, int stride, const std::vector<int>& there, int limit, unsigned seed) {
     Solve s(bps, nsys);
     for (int& k : s.link) k = -2;
@@ -107,6 +116,7 @@ int solve(int bps, int nsys, int stride, const std::vector<int>& there, int limi
             if (w.done(s)) live[at] = live.back(), live.pop_back();
         }
     }
+    if (s.spoiled) return -1;
     for (Group& w : g) most = w.walk.tries > most ? w.walk.tries : most;
     for (int k : there)
         for (int t = k; t < s.total; t += stride)
@@ -134,7 +144,7 @@ def run(tmp_path, main):
     return r.stdout
 
 
-@pytest.mark.parametrize("seeds", [[0], [1, 2, 3]])
+@pytest.mark.parametrize("seeds", [[0], [1, 2, 3], [4, 5, 6]])
 def test_every_tile_of_those_there_is_solved(tmp_path, seeds):
     out = run(tmp_path, r'''
 int main() {

@@ -168,6 +168,35 @@ def test_one_pass_sweeps_without_whole_groups(n, nsys, stride, parts, spin, refi
     test_one_pass_sweeps_that_are_not_all_there(n, nsys, stride, parts, spin, refine)
 
 
+@pytest.mark.parametrize("n,nsys,stride,parts,spin", [
+    (65536, 2, 16, [(0, 16)], 0),
+    (65536, 3, 5, [(0, 1), (1, 4)], 0),
+    (1 << 19, 2, 128, [(0, 128)], 0),
+    (1 << 19, 1, 128, [(0, 64), (64, 64)], 1),
+])
+def test_one_pass_answers_over_the_right_hand_sides(n, nsys, stride, parts, spin):
+    """x in d's own memory, with workgroups that publish each other's tiles:
+    the bits of a solve into memory of its own."""
+    say("in place", n, nsys, stride, parts, spin)
+    L = _diag()
+    a, b, c, d, _ = O.gen_batch(67, 0, nsys, n)
+    da, db, dc, dd = dev(a), dev(b), dev(c), dev(d)
+    ref = torch.zeros_like(dd)
+    B.solve_ex(da, db, dc, dd, ref, n, 256)
+    whole = dd.clone()
+    B.solve_ex(da, db, dc, whole, whole, n, 256)
+    assert np.array_equal(bits(whole), bits(ref))
+    ws = torch.empty(B.workspace_bytes(B.make_desc(da, db, dc, dd, ref, n, 256)), dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    p = ctypes.c_void_p
+    for i, (first, blocks) in enumerate(parts):
+        st = L.tprh_diag_split_fused(*(p(v.data_ptr()) for v in (da, db, dc, dd, dd)), n, nsys, 0, p(ws.data_ptr()),
+                                     int(i == 0), first, blocks, stride, spin, p(0))
+        assert st == 0
+        torch.cuda.synchronize()
+    assert np.array_equal(bits(dd), bits(ref))
+
+
 @pytest.mark.parametrize("refine", [False, True])
 @pytest.mark.parametrize("n,nsys,stride,first,blocks", [(65536, 2, 16, 0, 3), (1 << 17, 1, 32, 16, 2)])
 def test_one_pass_tile_given_up_is_nan(n, nsys, stride, first, blocks, refine):

@@ -48,6 +48,15 @@ __host__ __device__ __forceinline__ int fused_look(X& x, bool first, int ti, int
     }
 }
 
+// Whether a workgroup publishes the tile it has loaded.  seen: the tile was
+// published already when its loads were complete (asked for on behalf of
+// another workgroup only).  The answers of a system are stored once all its
+// tiles are published, so what was loaded before that are its inputs, even
+// where x is stored over d; after it, they may not be, and the words are there.
+__host__ __device__ inline bool fused_publishes(int kind, bool seen) {
+    return kind == kFusedOwn || (kind == kFusedHelp && !seen);
+}
+
 // Tasks that a workgroup can need beyond its own tiles, of which it has at
 // most total / stride, rounded up: each is taken up again, all other tiles of
 // its system are published, it is taken up once more; at the end there is no

@@ -160,6 +160,13 @@ __device__ __forceinline__ bool read_ends(const float* p4, const float* p2, Bloc
            b.x != kFusedEmpty && b.y != kFusedEmpty;
 }
 
+// s_seen of the wavefront: whether the tile with these words was published
+// when the wavefront's loads were complete.
+__device__ __forceinline__ void note_seen(const float* p2, int lane, int* s_seen) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(read_pair(p2)) ? 0 : 1;
+}
+
 // Polls until lanes with `need` have read their blocks' words into their e;
 // after `limit` polls gives up.  Returns the lanes still missing theirs.
 // Every lane of the wavefront calls this.
@@ -369,6 +376,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         float xo[E];
         unsigned long long seen = ~0ull;
         load_slices<E, HAS_B, CT>(loc, q, lo, run, stage, raw);
+        if (!REFINE && kind == kFusedHelp) note_seen(fw.ends2(ti), lane, s_seen);
         if constexpr (REFINE) {
             // No tile stores x before every tile of its system is published,
             // so x as loaded here is the iterate's if this tile (for the
@@ -424,9 +432,9 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         Chain16 ch;  // in every DPP row: lane l takes row l of the tile
         ch.reduce(BlockEnds{s_ends[0][l], s_ends[1][l], s_ends[2][l], s_ends[3][l], s_ends[4][l], s_ends[5][l]}, l);
         if (threadIdx.x < 64) {
-            const bool skip = REFINE && kind == kFusedHelp && (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
+            const bool there_before = kind == kFusedHelp && (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
             const BlockEnds mine = ch.ends(0);
-            if (threadIdx.x == 0 && kind != kFusedAgain && !skip) {
+            if (threadIdx.x == 0 && fused_publishes(kind, there_before)) {
                 if constexpr (REFINE) publish_pair(fw.x2(ti), xo[0], s_xlast);
                 publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
             }
