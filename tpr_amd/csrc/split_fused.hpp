@@ -115,8 +115,13 @@ struct BlockEnds {
     float fa, fc, fr, la, lc, lr;
 };
 
-// Two floats as published (a NaN of the empty pattern becomes another NaN),
+// A float, or two, as published (a NaN of the empty pattern becomes another NaN),
 // and back; missing: not published yet.
+__device__ __forceinline__ void publish_word(float* p, float x) {
+    const unsigned a = __builtin_bit_cast(unsigned, x);
+    __hip_atomic_store(reinterpret_cast<unsigned*>(p), a == kFusedEmpty ? 0x7fffffffu : a, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void publish_pair(float* p, float x, float y) {
     unsigned a = __builtin_bit_cast(unsigned, x), b = __builtin_bit_cast(unsigned, y);
     a = a == kFusedEmpty ? 0x7fffffffu : a;
@@ -351,7 +356,6 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
     __shared__ float s_ends[6][16];  // E_st and E_ed of the tile's rows
     __shared__ float s_side[2];      // x just before and just after the tile
     __shared__ int s_seen[4];        // per wavefront: the tile was published before it was loaded
-    __shared__ float s_xlast;        // the iterate's last x of the tile
     __shared__ int s_ok, s_tile, s_kind;
     const int bps = 1 << lg_bps;
     const int total = nsys << lg_bps;
@@ -374,7 +378,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         const size_t run = lo - (size_t)lane * E;
         RawPart<E> raw;
         float xo[E];
-        unsigned long long seen = ~0ull;
+        unsigned long long seen = ~0ull;  // in lane 0
         load_slices<E, HAS_B, CT>(loc, q, lo, run, stage, raw);
         if (!REFINE && kind == kFusedHelp) note_seen(fw.ends2(ti), lane, s_seen);
         if constexpr (REFINE) {
@@ -399,6 +403,14 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
                 }
             }
             residual_fp64<E, HAS_B>(xo, xl, xr, raw);
+            // x at the tile's ends, for whoever loads a tile beside it later:
+            // there before any of the words below (the wait ahead of the
+            // barrier) and so before any x of the tile is stored.  Not from a
+            // wavefront that loaded after the tile was published
+            if (kind != kFusedAgain && __ballot(!pair_missing(seen)) == 0) {
+                if (threadIdx.x == 0) publish_word(fw.x2(ti), xo[0]);
+                if (threadIdx.x == kFusedThreads - 1) publish_word(fw.x2(ti) + 1, xo[E - 1]);
+            }
         }
         RowState<METHOD, E> row;
         BlockEnds re;
@@ -415,7 +427,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         }
         if constexpr (REFINE) {
             if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(seen) ? 0 : 1;
-            if (threadIdx.x == kFusedThreads - 1) s_xlast = xo[E - 1];
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
         if constexpr (REFINE) {
@@ -434,10 +446,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         if (threadIdx.x < 64) {
             const bool there_before = kind == kFusedHelp && (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
             const BlockEnds mine = ch.ends(0);
-            if (threadIdx.x == 0 && fused_publishes(kind, there_before)) {
-                if constexpr (REFINE) publish_pair(fw.x2(ti), xo[0], s_xlast);
-                publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
-            }
+            if (threadIdx.x == 0 && fused_publishes(kind, there_before)) publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
             BlockEnds e{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             float before = 0.0f, after = 0.0f;
             bool there;  // every block that this tile waits for
