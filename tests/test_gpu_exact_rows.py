@@ -192,3 +192,40 @@ def test_tpr_shared_branches_bit_identical(E, L):
         assert bits_equal(x[k], ref[k]), k
     a, b, c, d, _ = O.gen_batch(78, 0, 5, n, O.GEN_WEAK)
     assert bits_equal(gpu(a, b, c, d, n, s, (E, L), method="tpr"), O.solve_batch("tpr", a, b, c, d, n, s))
+
+
+def zero_batch(seed, n, nsys):
+    """Systems whose off-diagonals and most right-hand sides are zeros of
+    either sign; the first is all +0 / -0 but for right-hand sides of -1."""
+    rng = np.random.default_rng(seed)
+
+    def pick(values):
+        return rng.choice(np.array(values, np.float32), nsys * n)
+
+    a, c = pick([0.0, -0.0]), pick([0.0, -0.0])
+    b, d = pick([1.0, 1.0, -1.0]), pick([0.0, -0.0, -0.0, 1.0, -1.0])
+    a[:n], c[:n], b[:n], d[:n] = 0.0, -0.0, 1.0, -1.0
+    d[0] = -0.0
+    return a, b, c, d
+
+
+@pytest.mark.parametrize("method", ["ptpr", "tpr"])
+@pytest.mark.parametrize("E,L", SHAPES)
+def test_signs_of_zeros_bit_identical(E, L, method):
+    """A missing partner must leave a right-hand side of -0 as it is."""
+    s = E * L
+    for m in (1, 2, 16):
+        n = s * m
+        if m * L > 1024:
+            continue
+        print("signs of zeros", method, E, L, m, flush=True)
+        a, b, c, d = zero_batch(75 + m, n, 20)
+        for diag in (b, np.ones_like(b)):
+            ref = O.solve_batch(method, a, diag, c, d, n, s)
+            assert bits_equal(gpu(a, diag, c, d, n, s, (E, L), method=method), ref)
+
+
+@pytest.mark.parametrize("n,s", [(32768, 128), (65536, 256), (65536, 2048)])
+def test_signs_of_zeros_multi_workgroup(n, s):
+    a, b, c, d = zero_batch(78, n, 3)
+    assert bits_equal(gpu(a, b, c, d, n, s), O.solve_batch("ptpr", a, b, c, d, n, s))

@@ -20,9 +20,10 @@
 //
 // The off-diagonals are kept negated (Ap = -a, Cp = -c), which changes no
 // rounding: in that form a missing partner is a product of +0 in the
-// denominator and the right-hand side and a factor 1 in the off-diagonal, so
-// the upper and lower formulas (src/ptpr.cpp:140-152, :171-182) take no
-// selects: the fused DPP products leave the lanes without a partner alone.
+// denominator, of -0 in the right-hand side (which may itself be -0, and
+// -0 + +0 would be +0) and a factor 1 in the off-diagonal, so the upper and
+// lower formulas (src/ptpr.cpp:140-152, :171-182) take no selects: the fused
+// DPP products leave the lanes without a partner alone.
 // A level's reciprocals share one range test and one wave-uniform branch.
 //
 // Measured (fp32 with a diagonal; the register form before -> this form ->
@@ -78,11 +79,12 @@ __device__ __forceinline__ void turn_blocked(float (&v)[E], float* area, int lan
     group_sync<true>();
 }
 
-// p = s(lane - D) * m and q = t(lane - D) * m, +0 in the first D lanes of the
-// slice.
+// p = s(lane - D) * m and q = t(lane - D) * m; +0 and -0 in the first D lanes
+// of the slice.
 template <int L, int D>
 __device__ __forceinline__ void exact_mul_up(float s, float t, float m, int l, float& p, float& q) {
-    p = q = 0.0f;
+    p = 0.0f;
+    q = -0.0f;
     if constexpr (L == 16) {
         asm("s_nop 1\n\t"
             "v_mul_f32_dpp %[p], %[s], %[m] row_shr:%[d] row_mask:0xf bank_mask:0xf\n\t"
@@ -92,13 +94,14 @@ __device__ __forceinline__ void exact_mul_up(float s, float t, float m, int l, f
     } else {
         const float x = shift_up<L, D>(s, 0.0f, l) * m, y = shift_up<L, D>(t, 0.0f, l) * m;
         p = l >= D ? x : 0.0f;
-        q = l >= D ? y : 0.0f;
+        q = l >= D ? y : -0.0f;
     }
 }
-// The same from lane + D, +0 in the last D lanes.
+// The same from lane + D, +0 and -0 in the last D lanes.
 template <int L, int D>
 __device__ __forceinline__ void exact_mul_dn(float s, float t, float m, int l, float& p, float& q) {
-    p = q = 0.0f;
+    p = 0.0f;
+    q = -0.0f;
     if constexpr (L == 16) {
         asm("s_nop 1\n\t"
             "v_mul_f32_dpp %[p], %[s], %[m] row_shl:%[d] row_mask:0xf bank_mask:0xf\n\t"
@@ -108,7 +111,7 @@ __device__ __forceinline__ void exact_mul_dn(float s, float t, float m, int l, f
     } else {
         const float x = shift_down<L, D>(s, 0.0f, l) * m, y = shift_down<L, D>(t, 0.0f, l) * m;
         p = l < L - D ? x : 0.0f;
-        q = l < L - D ? y : 0.0f;
+        q = l < L - D ? y : -0.0f;
     }
 }
 // s(lane - D) * u, or u in the first D lanes; s(lane + D) * u, or u in the
