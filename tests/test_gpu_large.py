@@ -174,6 +174,40 @@ def test_refinement_step_bit_identical(method, n, s, nsys):
     assert bits_equal(x1, oracle_refine(method, a, b, c, d, x0, n, s))
 
 
+@pytest.mark.parametrize("arith", ["exact", "fast"])
+@pytest.mark.parametrize("method", ["ptpr", "tpr"])
+@pytest.mark.parametrize("n,nsys", [(2048, 5), (4096, 3), (16384, 3), (32768, 3)])
+def test_32_equations_per_lane(method, arith, n, nsys):
+    """s = 2048 on 32 x 64 slices, loads and stores through LDS: one wavefront
+    per system up to the largest of one workgroup (1024 lanes), with a diagonal
+    and without, fp16 storage, a shared matrix and a refinement step, and
+    nothing written past x."""
+    say("32 per lane", method, arith, n, nsys)
+    s = 2048
+    a, b, c, d, _ = O.gen_batch(38, 0, nsys, n, O.GEN_WEAK if arith == "exact" else O.GEN_DOMINANT)
+    one = np.ones_like(b)
+    h = [v.astype(np.float16) for v in (a, b, c)]
+    x0 = O.solve_batch(method, a, b, c, d, n, s) * np.float32(1.001)
+    first = [np.tile(v[:n], nsys) for v in (a, b, c)]
+    cases = [("diagonal", (a, b, c), {}, O.solve_batch(method, a, b, c, d, n, s)),
+             ("unit", (a / b, None, c / b), {}, O.solve_batch(method, a / b, one, c / b, d, n, s)),
+             ("fp16", h, {}, O.solve_batch(method, *(v.astype(np.float32) for v in h), d, n, s)),
+             ("shared", [v[:n] for v in (a, b, c)], {"shared": True}, O.solve_batch(method, *first, d, n, s)),
+             ("refine", (a, b, c), {"refine": True}, oracle_refine(method, a, b, c, d, x0, n, s))]
+    for name, coef, kw, ref in cases:
+        coef = [None if v is None else dev(v, torch.float16 if v.dtype == np.float16 else torch.float32) for v in coef]
+        x = torch.full((nsys * n + 4096,), 2.5, device="cuda")
+        x[:nsys * n] = dev(x0)
+        B.solve_ex(*coef, dev(d), x[:nsys * n], n, s, method=method, arith=arith, shape=(32, 64), **kw)
+        torch.cuda.synchronize()
+        assert bool((x[nsys * n:] == 2.5).all()), name
+        x = x[:nsys * n].cpu().numpy()
+        if arith == "exact":
+            assert bits_equal(x, ref), name
+        else:
+            assert per_system_rel(x, ref, n).max() <= FAST_TOL, name
+
+
 @pytest.mark.parametrize("method", ["ptpr", "tpr"])
 def test_refinement_reaches_fp64_accuracy(method):
     """Weakly dominant systems (the `weak` generator, smaller n): the fp16-stored
