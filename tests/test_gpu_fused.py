@@ -76,6 +76,27 @@ def test_one_pass_forms_agree(method, n, s, nsys):
         assert rel(one.cpu().numpy(), two.cpu().numpy(), n) <= FAST_TOL, kw
 
 
+@pytest.mark.parametrize("n,s,nsys", [(1 << 20, 512, 2), (1 << 21, 1024, 1)])
+@pytest.mark.parametrize("method", ["ptpr", "tpr"])
+def test_one_pass_refinement_with_many_groups(method, n, s, nsys):
+    """A refinement step in the one-pass form on 256 and 512 tiles per system.
+    (At three workgroups per CU the device does not hold the 1024 tiles of 4
+    Mi equations at once, and that step takes two passes.)"""
+    say("one pass, many groups", method, n, s, nsys)
+    a, b, c, d, _ = O.gen_batch(68, 0, nsys, n)
+    da, db, dc, dd = dev(a), dev(b), dev(c), dev(d)
+    ref = O.thomas_f64_batch(a, b, c, d, n)
+    start = dev(O.solve_batch(method, a, b, c, d, n, s)) * 1.001
+    err = []
+    for form in (0, 1):
+        x = start.clone()
+        B.solve_ex(da, db, dc, dd, x, n, s, split_form=form, method=method, refine=True)
+        torch.cuda.synchronize()
+        err.append(rel(x.cpu().numpy(), ref, n))
+    say(err)
+    assert err[0] <= max(2 * err[1], 1e-7)
+
+
 @pytest.mark.parametrize("n,s,nsys", [(65536, 256, 70), (524288, 512, 9)])
 @pytest.mark.parametrize("method", ["ptpr", "tpr"])
 def test_one_pass_weakly_dominant_accuracy(method, n, s, nsys):
