@@ -138,22 +138,27 @@ tprh_status tprh_solve_batched(tprh_method method, tprh_arith arith, const float
 
 /* Same with an explicit slice shape: E equations per lane, L lanes per slice
  * (E * L == s).  Used by the autotuner; tprh_shape_supported() lists what is
- * compiled in. */
+ * compiled in.  Exact answers are the same bits with every shape; fast
+ * answers of two shapes may differ in rounding.  In fast PTPR the shapes 16 x
+ * 32, 16 x 64 and (up to n = 16384) 32 x 64 are run as rows of 16 lanes x 16
+ * equations, n / 256 of them, with the answers of s = 256: the slice's
+ * interior may be eliminated in any order there, and this one is faster. */
 tprh_status tprh_solve_batched_shape(tprh_method method, tprh_arith arith, const float *a, const float *b,
                                      const float *c, const float *d, float *x, int n, int s, int nsys,
                                      int E, int L, void *stream);
 int tprh_shape_supported(int E, int L);
 /* The slice shape (E equations per lane, L lanes per slice) that
- * tprh_solve_batched takes for this method, arithmetic, n, s and batch size;
- * no device call.  Errors as tprh_solve_batched's for (n, s). */
+ * tprh_solve_batched takes for this method, arithmetic, n, s and batch size
+ * (as tprh_solve_batched_shape takes it: fast PTPR's 16 x 32, 16 x 64 and 32 x
+ * 64 are run as said there); no device call.  Errors as tprh_solve_batched's for (n, s). */
 tprh_status tprh_slice_shape(tprh_method method, tprh_arith arith, int n, int s, int nsys, int *E, int *L);
 
 /* ---- the general entry point ---------------------------------------------
  * Everything tprh_solve_batched does, plus:
  *   - systems larger than one workgroup (n / s * L > 1024 lanes, up to 2048
- *     slices per system): solved in rounds of `chunk` systems by three
- *     kernels (stage 1, reduced system, stage 3) through a caller-provided
- *     workspace of tprh_workspace_bytes(desc) bytes (device memory);
+ *     slices per system): solved in rounds of `chunk` systems, in one of the
+ *     forms of split_form below, through a caller-provided workspace of
+ *     tprh_workspace_bytes(desc) bytes (device memory);
  *   - coefficients a, b, c stored as fp16 (TPRH_STORE_F16; d and x stay fp32;
  *     the solve computes in fp32);
  *   - one iterative-refinement step (refine = 1): x += A^-1 (d - A x) with the

@@ -57,7 +57,8 @@ def _stream(stream):
 def solve_batched(a, b, c, d, x, n, s, method="ptpr", arith="fast", shape=None, stream=None):
     """Solve nsys = numel // n systems; b may be None (unit diagonal).
 
-    shape: optional (E, L) slice shape (equations per lane, lanes per slice).
+    shape: optional (E, L) slice shape (equations per lane, lanes per slice;
+    fast PTPR runs 16 x 32, 16 x 64 and 32 x 64 as rows of 16 x 16).
     """
     nsys = a.numel() // n
     tot = nsys * n

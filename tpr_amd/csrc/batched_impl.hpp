@@ -111,7 +111,8 @@ hipError_t launch_b(const BatchArgs& p, int grid, int block, size_t shmem, int l
     auto* kern = p.b != nullptr ? batched_kernel<METHOD, E, L, MODE, BLOCK, true, CT, REFINE>
                                 : batched_kernel<METHOD, E, L, MODE, BLOCK, false, CT, REFINE>;
     if (shmem > 65536) {
-        // 1024-lane systems of 16 equations per lane stage 68 KB
+        // with their systems' rows, 1024-lane workgroups stage 68 KB at 16
+        // equations per lane and 136 at 32, 512-lane ones 68 at 32
         static std::atomic<unsigned long long> set_b{0}, set_u{0};
         hipError_t e = ensure_lds_limit(reinterpret_cast<const void*>(kern), (int)shmem, p.b != nullptr ? set_b : set_u);
         if (e != hipSuccess) return e;

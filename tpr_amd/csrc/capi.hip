@@ -358,8 +358,8 @@ bool answers_arrived(const float* x, int n) {
 
 // Systems up to this many equations are solved straight from the mapped
 // pinned buffer: the kernel reads a, c, rhs (and diag) over the host link
-// and writes x back the same way, so a call is one launch and one stream
-// synchronisation, with no copy engine in between.  Larger systems (and the
+// and writes x back the same way, so a call is one launch and a wait for the
+// answers, with no copy engine in between.  Larger systems (and the
 // multi-workgroup path) are copied to device memory first.
 constexpr int kZeroCopyMaxN = 1 << 16;
 

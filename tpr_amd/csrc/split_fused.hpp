@@ -6,8 +6,8 @@
 // rate such bytes can be moved (K1 46, K2 6, K3 47 us); reading the inputs
 // once leaves 336 MB.  A whole solve of that batch: 101 us two passes, 63.5
 // us this way (5.3 TB/s; a device copy of that size reaches 4.8-5.4); with an
-// fp16-stored solve and a refinement step 203 -> 129 us; one system of 1 Mi
-// equations 29 -> 14 us.
+// fp16-stored solve and a refinement step 203 -> 130 us; one system of 1 Mi
+// equations 29.4 -> 11.4 us.
 //
 // A tile is 4096 consecutive equations of one system: 256 lanes x 16, sixteen
 // rows of 16 lanes (one DPP row, 256 equations).  A workgroup
