@@ -73,10 +73,14 @@ struct Group {  // a workgroup
         } else if (ti % kFusedGroup != 0 && kind == kFusedOwn) {
             ok = s.result[tile];
         } else {
-            const int lost = fused_look(w, kind == kFusedOwn, ti, 0);
-            ok = lost < 0;
-            if (!ok) missing = base + lost;
-            else for (int k = 0; k < kFusedGroup; k++) s.result[tile / kFusedGroup * kFusedGroup + k] = 1;
+            const int g = ti / kFusedGroup, lost = kind != kFusedOwn ? fused_look(w, ti, 0) : -1;
+            ok = lost < 0 && w.tiles(g, 0) == 0;
+            if (ok) {
+                w.publish(g);
+                ok = w.groups(0) == 0;
+            }
+            missing = base + lost;
+            if (ok) for (int k = 0; k < kFusedGroup; k++) s.result[tile / kFusedGroup * kFusedGroup + k] = 1;
         }
         if (!ok && kind == kFusedOwn && patient) return;
         step = 0;

@@ -22,28 +22,23 @@ __host__ __device__ inline int fused_pick(unsigned long long missing, int from) 
     return __builtin_ctzll(above ? above : missing);
 }
 
-// Systems of more than 16 tiles: -1 once every group's words are there for
-// tile ti, else a tile (in the system) that is missing.  x.tiles(g, limit)
-// and x.groups(limit) poll up to `limit` more times for the 16 tiles of group
-// g and for the groups, and return which are missing; x.publish(g) publishes
-// group g from the tiles just read.  A tile waiting for the first time
-// (`first`) only asks; afterwards a group whose tiles are all there, but
-// whose first tile's workgroup is not, is published here, so that what is
-// returned is always a tile not yet published when it was looked at.
+// Systems of more than 16 tiles, for a workgroup that has waited for tile ti
+// in vain: -1 once every tile and every group is published, else a tile (in
+// the system) that was missing when it was looked at.  x.tiles(g, limit) and
+// x.groups(limit) poll up to `limit` more times for the 16 tiles of group g
+// and for the groups, and return which are missing; x.publish(g) publishes
+// group g from the tiles just read: a group whose tiles are all there, but
+// whose first tile's workgroup is not, is published here.
 template <typename X>
-__host__ __device__ __forceinline__ int fused_look(X& x, bool first, int ti, int limit) {
-    const int g = ti / kFusedGroup;
-    unsigned long long m = x.tiles(g, limit);
-    if (m != 0) return g * kFusedGroup + fused_pick(m, ti % kFusedGroup);
-    x.publish(g);
-    for (;;) {  // ends: each turn but the last publishes a missing group
+__host__ __device__ __forceinline__ int fused_look(X& x, int ti, int limit) {
+    const int own = ti / kFusedGroup;
+    for (int g = own;;) {  // ends: each turn publishes a missing group
+        unsigned long long m = x.tiles(g, limit);
+        if (m != 0) return g * kFusedGroup + fused_pick(m, ti % kFusedGroup);
+        x.publish(g);
         m = x.groups(limit);
         if (m == 0) return -1;
-        const int other = fused_pick(m, g);
-        if (first) return other * kFusedGroup;
-        m = x.tiles(other, 0);
-        if (m != 0) return other * kFusedGroup + fused_pick(m, ti % kFusedGroup);
-        x.publish(other);
+        g = fused_pick(m, own);
         limit = 0;
     }
 }

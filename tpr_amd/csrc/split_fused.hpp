@@ -318,9 +318,8 @@ struct RowState<1, E> {  // TPR: the tree (src/tpr.cpp:123-230, :277-308)
 // What a wavefront reads and publishes of a system of groups (fused_look).
 struct GroupWords {
     const FusedWords fw;
-    const int lane, own;  // own: the tile's group
-    BlockEnds e;          // of the blocks last read, one per lane; past the last one zero equations
-    Chain16 chain;        // of the own group, once published
+    const int lane;
+    BlockEnds e;  // of the blocks last read, one per lane; past the last one zero equations
 
     __device__ __forceinline__ unsigned long long tiles(int g, int limit) {
         const int t = g * kFusedGroup + (lane & 15);
@@ -331,12 +330,12 @@ struct GroupWords {
         e = BlockEnds{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         return wait_ends(fw.group4(lane), fw.group2(lane), lane < fw.groups(), limit, e);
     }
-    __device__ __forceinline__ void publish(int g) {
+    __device__ __forceinline__ Chain16 publish(int g) {
         Chain16 c;
         c.reduce(e, lane & 15);
         const BlockEnds ge = c.ends(0);
         if (lane == 0) publish_ends(fw.group4(g), fw.group2(g), ge);
-        if (g == own) chain = c;
+        return c;
     }
 };
 
@@ -380,7 +379,6 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         float xo[E];
         unsigned long long seen = ~0ull;  // in lane 0
         load_slices<E, HAS_B, CT>(loc, q, lo, run, stage, raw);
-        if (!REFINE && kind == kFusedHelp) note_seen(fw.ends2(ti), lane, s_seen);
         if constexpr (REFINE) {
             // No tile stores x before every tile of its system is published,
             // so x as loaded here is the iterate's if this tile (for the
@@ -403,14 +401,6 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
                 }
             }
             residual_fp64<E, HAS_B>(xo, xl, xr, raw);
-            // x at the tile's ends, for whoever loads a tile beside it later:
-            // there before any of the words below (the wait ahead of the
-            // barrier) and so before any x of the tile is stored.  Not from a
-            // wavefront that loaded after the tile was published
-            if (kind != kFusedAgain && __ballot(!pair_missing(seen)) == 0) {
-                if (threadIdx.x == 0) publish_word(fw.x2(ti), xo[0]);
-                if (threadIdx.x == kFusedThreads - 1) publish_word(fw.x2(ti) + 1, xo[E - 1]);
-            }
         }
         RowState<METHOD, E> row;
         BlockEnds re;
@@ -426,8 +416,18 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             s_ends[5][j] = re.lr;
         }
         if constexpr (REFINE) {
+            // x at the tile's ends, for whoever loads a tile beside it later:
+            // there before any of the words below (the wait ahead of the
+            // barrier) and so before any x of the tile is stored.  Not from a
+            // wavefront that loaded after the tile was published
+            if (kind != kFusedAgain && __ballot(!pair_missing(seen)) == 0) {
+                if (threadIdx.x == 0) publish_word(fw.x2(ti), xo[0]);
+                if (threadIdx.x == kFusedThreads - 1) publish_word(fw.x2(ti) + 1, xo[E - 1]);
+            }
             if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(seen) ? 0 : 1;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else if (__builtin_expect(kind == kFusedHelp, 0)) {
+            note_seen(fw.ends2(ti), lane, s_seen);
         }
         __syncthreads();
         if constexpr (REFINE) {
@@ -454,7 +454,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             if constexpr (!WIDE) {
                 const unsigned long long m = wait_ends(fw.ends4(lane), fw.ends2(lane), lane < bps, limit, e);
                 there = m == 0;
-                if (there) solve_blocks<false>(e, bps, ti, lane, before, after);
+                if (__builtin_expect(there, 1)) solve_blocks<false>(e, bps, ti, lane, before, after);
                 else missing = tile - ti + fused_pick(m, ti);
             } else if (ti % kFusedGroup != 0 && kind == kFusedOwn) {
                 there = wait_pair(fw.result(ti), lane, limit, before, after) == 0;
@@ -463,19 +463,23 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
                 // of the groups and hands every tile of the group its sides
                 // (a tile taken up again does so by itself)
                 const int g = ti / kFusedGroup;
-                GroupWords gw{fw, lane, g};
-                const int lost = fused_look(gw, kind == kFusedOwn, ti, limit);
-                there = lost < 0;
+                GroupWords gw{fw, lane};
+                int lost = -1;
+                if (__builtin_expect(kind != kFusedOwn, 0)) lost = fused_look(gw, ti, limit);
+                there = lost < 0 && gw.tiles(g, limit) == 0;
                 if (there) {
-                    float ob, oa, xb, xe, xa;
-                    solve_blocks<true>(gw.e, fw.groups(), g, lane, ob, oa);
-                    gw.chain.solve(ob, oa, l, xb, xe, xa);
-                    if (lane < kFusedGroup) publish_pair(fw.result(g * kFusedGroup + l), xb, xa);
-                    before = __shfl(xb, ti % kFusedGroup, 64);
-                    after = __shfl(xa, ti % kFusedGroup, 64);
-                } else {
-                    missing = tile - ti + lost;
+                    const Chain16 chain = gw.publish(g);
+                    there = gw.groups(limit) == 0;
+                    if (there) {
+                        float ob, oa, xb, xe, xa;
+                        solve_blocks<true>(gw.e, fw.groups(), g, lane, ob, oa);
+                        chain.solve(ob, oa, l, xb, xe, xa);
+                        if (lane < kFusedGroup) publish_pair(fw.result(g * kFusedGroup + l), xb, xa);
+                        before = __shfl(xb, ti % kFusedGroup, 64);
+                        after = __shfl(xa, ti % kFusedGroup, 64);
+                    }
                 }
+                missing = tile - ti + lost;
             }
             if (threadIdx.x == 0) {
                 const bool lost = !there && kind == kFusedAgain && walk.lost(tasks);  // its x: NaN
@@ -486,7 +490,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         }
         __syncthreads();
         const bool ok = __builtin_amdgcn_readfirstlane(s_ok) != 0;
-        if (ok && kind != kFusedHelp) {
+        if (__builtin_expect(ok && kind != kFusedHelp, 1)) {
             float xb, xe, xa;
             ch.solve(s_side[0], s_side[1], l, xb, xe, xa);
             const int src = (lane & 48) + j;  // a lane that holds row j
