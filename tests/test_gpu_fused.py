@@ -284,3 +284,36 @@ def test_one_pass_in_a_graph_and_on_streams():
     torch.cuda.synchronize()
     for t, e in zip(sets, eager):
         assert np.array_equal(bits(t["x"]), e)
+
+
+def _masked_stream(cus):
+    """A stream of default priority on the device's first `cus` CUs."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    torch.zeros(1, device="cuda")
+    words = (ctypes.c_uint32 * ((cus + 31) // 32))(*[(1 << min(32, cus - k)) - 1 for k in range(0, cus, 32)])
+    st = ctypes.c_void_p()
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(st), len(words), words) == 0
+    return torch.cuda.ExternalStream(st.value), lambda: hip.hipStreamDestroy(st)
+
+
+@pytest.mark.parametrize("refine", [False, True])
+@pytest.mark.parametrize("n,s,nsys,form", [(65536, 256, 20, 0), (1 << 20, 512, 1, 1)])
+def test_one_pass_on_a_stream_with_a_cu_mask(n, s, nsys, form, refine):
+    """On 32 CUs: systems that their workgroups hold at once take one pass,
+    larger ones two (form: whose bits, on the whole device, the answers are)."""
+    say("CU mask", n, s, nsys, refine)
+    t = B.alloc_batch(nsys, n)
+    B.generate("dominant", 69, 0, nsys, n, t["a"], t["b"], t["c"], t["d"], t["xt"])
+    args = (t["a"], t["b"], t["c"], t["d"], t["x"], n, s)
+    ws = torch.empty(B.workspace_bytes(B.make_desc(*args)), dtype=torch.uint8, device="cuda")
+    got = {}
+    st, destroy = _masked_stream(32)
+    for name, f, stream in (("one", 0, None), ("two", 1, None), ("masked", 0, st)):
+        t["x"].copy_(t["xt"] * 1.001)
+        torch.cuda.synchronize()
+        B.solve_ex(*args, refine=refine, split_form=f, workspace=ws, stream=stream)
+        torch.cuda.synchronize()
+        got[name] = bits(t["x"])
+    destroy()
+    assert not np.array_equal(got["one"], got["two"])
+    assert np.array_equal(got["masked"], got["two" if form else "one"])

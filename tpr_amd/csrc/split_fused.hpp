@@ -535,23 +535,43 @@ int resident_workgroups(K kernel, int threads, size_t lds) {
     return cus * occ;
 }
 
+// CUs that a stream's kernels run on, of the device's `cus`: fewer on a stream
+// made with a CU mask (0.2 us on the host).
+inline int stream_cus(hipStream_t stream, int cus) {
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(stream, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return cus;
+    }
+    int n = 0;
+    for (uint32_t w : mask) n += __builtin_popcount(w);
+    return n > 0 && n < cus ? n : cus;
+}
+
 template <int METHOD, bool HAS_B, typename CT, bool REFINE, bool WIDE, typename Loc>
 hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, bool* done) {
     const int lg_bps = __builtin_ctz((unsigned)(n / kFusedTile));
     const auto kern = fused_split_kernel<METHOD, HAS_B, CT, REFINE, WIDE, Loc>;
-    // workgroups resident at once, asked once per device: the query costs
-    // the host as much as a launch
-    static std::atomic<int> known[64];
+    // workgroups resident at once: those of a CU and the CUs, asked once per
+    // device (the query costs the host as much as a launch), times the
+    // stream's share of the CUs
+    static std::atomic<int> known_cus[64], known_all[64];
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    int capacity = dev < 64 ? known[dev].load(std::memory_order_relaxed) : 0;
-    if (capacity == 0) {
-        // a multiple of the group, so that a system's tiles run side by side
-        // in every sweep of the grid over the tiles
-        capacity = resident_workgroups(kern, kFusedThreads, 0) & ~(kFusedGroup - 1);
-        if (dev < 64) known[dev].store(capacity, std::memory_order_relaxed);
+    int cus = dev < 64 ? known_cus[dev].load(std::memory_order_acquire) : 0;
+    int all = cus ? known_all[dev].load(std::memory_order_relaxed) : 0;
+    if (cus == 0) {
+        all = resident_workgroups(kern, kFusedThreads, 0);
+        if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+        if (dev < 64) {
+            known_all[dev].store(all, std::memory_order_relaxed);
+            known_cus[dev].store(cus, std::memory_order_release);
+        }
     }
+    // a multiple of the group, so that a system's tiles run side by side in
+    // every sweep of the grid over the tiles
+    const int capacity = (int)((long long)all * stream_cus(stream, cus) / cus) & ~(kFusedGroup - 1);
     *done = capacity >= 1 << lg_bps;
     if (!*done) return hipSuccess;
     const int tiles = nsys << lg_bps;
@@ -565,10 +585,11 @@ hipError_t launch_fused_t(const Loc& loc, int n, int nsys, hipStream_t stream, b
 }
 
 // One round: nsys systems of n equations (n / kFusedTile tiles each) at loc.
-// *done is false, and nothing is launched, where the device does not hold a
-// whole system's workgroups at once (a refinement step on 4 Mi equations, at
-// three workgroups per CU): every tile would be loaded twice (4 Mi equations:
-// 104 us that way, 97 in two passes).
+// *done is false, and nothing is launched, where the stream's CUs do not hold
+// a whole system's workgroups at once (a refinement step on 4 Mi equations, at
+// three workgroups per CU; a stream with a CU mask): every tile would be
+// loaded twice or more (4 Mi equations: 104 us that way, 97 in two passes; 1
+// Mi on 32 CUs 478, 87).
 template <int METHOD, bool HAS_B, typename CT, bool REFINE, typename Loc>
 hipError_t launch_fused(const Loc& loc, int n, int nsys, hipStream_t stream, bool* done) {
     return n / kFusedTile > kFusedGroup ? launch_fused_t<METHOD, HAS_B, CT, REFINE, true>(loc, n, nsys, stream, done)
