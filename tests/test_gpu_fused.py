@@ -10,6 +10,7 @@ the FP64 Thomas solve, or 1e-6.
 import ctypes
 import os
 import sys
+import types
 
 import numpy as np
 import pytest
@@ -317,3 +318,22 @@ def test_one_pass_on_a_stream_with_a_cu_mask(n, s, nsys, form, refine):
     destroy()
     assert not np.array_equal(got["one"], got["two"])
     assert np.array_equal(got["masked"], got["two" if form else "one"])
+
+
+@pytest.mark.parametrize("handle", [0, 1, 2])
+def test_one_pass_on_the_null_streams(handle):
+    """The null stream by its handles (default, legacy, per thread)."""
+    say("null stream", handle)
+    n, nsys = 65536, 2
+    t = B.alloc_batch(nsys, n)
+    B.generate("dominant", 70, 0, nsys, n, t["a"], t["b"], t["c"], t["d"], t["xt"])
+    args = (t["a"], t["b"], t["c"], t["d"], t["x"], n, 256)
+    ws = torch.empty(B.workspace_bytes(B.make_desc(*args)), dtype=torch.uint8, device="cuda")
+    B.solve_ex(*args, workspace=ws)
+    torch.cuda.synchronize()
+    want = bits(t["x"])
+    t["x"].zero_()
+    torch.cuda.synchronize()
+    B.solve_ex(*args, workspace=ws, stream=types.SimpleNamespace(cuda_stream=handle))
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(t["x"]), want)
