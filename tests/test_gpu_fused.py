@@ -17,6 +17,7 @@ import pytest
 import torch
 
 import oracle as O
+from tpr_amd import _lib
 from tpr_amd import batched as B
 from tpr_amd import build
 
@@ -337,3 +338,24 @@ def test_one_pass_on_the_null_streams(handle):
     B.solve_ex(*args, workspace=ws, stream=types.SimpleNamespace(cuda_stream=handle))
     torch.cuda.synchronize()
     assert np.array_equal(bits(t["x"]), want)
+
+
+def test_one_pass_refuses_a_destroyed_stream():
+    """As a launch does: an error, before anything runs."""
+    say("destroyed stream")
+    n, nsys = 65536, 2
+    t = B.alloc_batch(nsys, n)
+    B.generate("dominant", 71, 0, nsys, n, t["a"], t["b"], t["c"], t["d"], t["xt"])
+    args = (t["a"], t["b"], t["c"], t["d"], t["x"], n, 256)
+    ws = torch.empty(B.workspace_bytes(B.make_desc(*args)), dtype=torch.uint8, device="cuda")
+    t["x"].fill_(2.5)
+    st, destroy = _masked_stream(64)
+    torch.cuda.synchronize()
+    assert destroy() == 0
+    with pytest.raises(_lib.TprError):
+        B.solve_ex(*args, workspace=ws, stream=types.SimpleNamespace(cuda_stream=st.cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((t["x"] == 2.5).all())
+    B.solve_ex(*args, workspace=ws)
+    torch.cuda.synchronize()
+    assert rel(t["x"].cpu().numpy(), t["xt"].cpu().numpy(), n) <= FAST_TOL

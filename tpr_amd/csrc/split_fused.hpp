@@ -536,11 +536,14 @@ int resident_workgroups(K kernel, int threads, size_t lds) {
 }
 
 // CUs that a stream's kernels run on, of the device's `cus`: fewer on a stream
-// made with a CU mask (0.2 us on the host).  The query takes no legacy handle
-// for the null stream.
+// made with a CU mask (0.3 us on the host).  The mask query takes neither the
+// null stream's legacy handle nor a stream destroyed, which the launch refuses.
 inline int stream_cus(hipStream_t stream, int cus) {
     uint32_t mask[32] = {};
-    if (hipExtStreamGetCUMask(stream == hipStreamLegacy ? nullptr : stream, 32, mask) != hipSuccess) {
+    hipDevice_t dev;
+    if (stream == hipStreamLegacy) stream = nullptr;
+    if ((stream && hipStreamGetDevice(stream, &dev) != hipSuccess) ||
+        hipExtStreamGetCUMask(stream, 32, mask) != hipSuccess) {
         (void)hipGetLastError();
         return cus;
     }
