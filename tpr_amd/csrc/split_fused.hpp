@@ -6,7 +6,7 @@
 // rate such bytes can be moved (K1 46, K2 6, K3 47 us); reading the inputs
 // once leaves 336 MB.  A whole solve of that batch: 101 us two passes, 63.5
 // us this way (5.3 TB/s; a device copy of that size reaches 4.8-5.4); with an
-// fp16-stored solve and a refinement step 203 -> 130 us; one system of 1 Mi
+// fp16-stored solve and a refinement step 203 -> 127.5 us; one system of 1 Mi
 // equations 29.4 -> 11.4 us.
 //
 // A tile is 4096 consecutive equations of one system: 256 lanes x 16, sixteen
@@ -115,13 +115,8 @@ struct BlockEnds {
     float fa, fc, fr, la, lc, lr;
 };
 
-// A float, or two, as published (a NaN of the empty pattern becomes another NaN),
+// Two floats as published (a NaN of the empty pattern becomes another NaN),
 // and back; missing: not published yet.
-__device__ __forceinline__ void publish_word(float* p, float x) {
-    const unsigned a = __builtin_bit_cast(unsigned, x);
-    __hip_atomic_store(reinterpret_cast<unsigned*>(p), a == kFusedEmpty ? 0x7fffffffu : a, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ void publish_pair(float* p, float x, float y) {
     unsigned a = __builtin_bit_cast(unsigned, x), b = __builtin_bit_cast(unsigned, y);
     a = a == kFusedEmpty ? 0x7fffffffu : a;
@@ -163,13 +158,6 @@ __device__ __forceinline__ bool read_ends(const float* p4, const float* p2, Bloc
     e = BlockEnds{f(a.x), f(a.y), f(a.z), f(a.w), f(b.x), f(b.y)};
     return a.x != kFusedEmpty && a.y != kFusedEmpty && a.z != kFusedEmpty && a.w != kFusedEmpty &&
            b.x != kFusedEmpty && b.y != kFusedEmpty;
-}
-
-// s_seen of the wavefront: whether the tile with these words was published
-// when the wavefront's loads were complete.
-__device__ __forceinline__ void note_seen(const float* p2, int lane, int* s_seen) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(read_pair(p2)) ? 0 : 1;
 }
 
 // Polls until lanes with `need` have read their blocks' words into their e;
@@ -378,6 +366,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         RawPart<E> raw;
         float xo[E];
         unsigned long long seen = ~0ull;  // in lane 0
+        float tile_end = 0.0f;            // refinement: the iterate's last x of the tile, in thread 0
         load_slices<E, HAS_B, CT>(loc, q, lo, run, stage, raw);
         if constexpr (REFINE) {
             // No tile stores x before every tile of its system is published,
@@ -388,7 +377,14 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             load_e<E>(loc.X(q) + lo, xo);
             float xl, xr;
             wave_halo<E>(loc.X(q), lo, loc.n, lane, xo, xl, xr);
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the loads are complete before the reads below
+            if (threadIdx.x == 0) tile_end = loc.X(q)[lo + kFusedTile - 1];
+            // the loads are complete before the reads below (xl and xr: the
+            // compiler would else wait for them, and so for all of those, where
+            // the values are used)
+            asm volatile("s_waitcnt vmcnt(0)" : "+v"(xl), "+v"(xr), "+v"(tile_end)::"memory");
+            // x at the tile's ends, for whoever loads a tile beside it later.
+            // An own tile's x is the iterate's until this workgroup stores it
+            if (threadIdx.x == 0 && kind == kFusedOwn) publish_pair(fw.x2(ti), xo[0], tile_end);
             if (lane == 0) seen = read_pair(fw.ends2(ti));
             if (kind != kFusedOwn) {
                 if (threadIdx.x == 0 && ti > 0) {
@@ -416,18 +412,7 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
             s_ends[5][j] = re.lr;
         }
         if constexpr (REFINE) {
-            // x at the tile's ends, for whoever loads a tile beside it later:
-            // there before any of the words below (the wait ahead of the
-            // barrier) and so before any x of the tile is stored.  Not from a
-            // wavefront that loaded after the tile was published
-            if (kind != kFusedAgain && __ballot(!pair_missing(seen)) == 0) {
-                if (threadIdx.x == 0) publish_word(fw.x2(ti), xo[0]);
-                if (threadIdx.x == kFusedThreads - 1) publish_word(fw.x2(ti) + 1, xo[E - 1]);
-            }
             if (lane == 0) s_seen[threadIdx.x >> 6] = pair_missing(seen) ? 0 : 1;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        } else if (__builtin_expect(kind == kFusedHelp, 0)) {
-            note_seen(fw.ends2(ti), lane, s_seen);
         }
         __syncthreads();
         if constexpr (REFINE) {
@@ -444,9 +429,21 @@ __global__ __launch_bounds__(kFusedThreads, REFINE ? 3 : 4) void fused_split_ker
         Chain16 ch;  // in every DPP row: lane l takes row l of the tile
         ch.reduce(BlockEnds{s_ends[0][l], s_ends[1][l], s_ends[2][l], s_ends[3][l], s_ends[4][l], s_ends[5][l]}, l);
         if (threadIdx.x < 64) {
-            const bool there_before = kind == kFusedHelp && (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
             const BlockEnds mine = ch.ends(0);
-            if (threadIdx.x == 0 && fused_publishes(kind, there_before)) publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
+            bool there_before = false;  // of a tile of another's: published when all its loads were complete
+            if (threadIdx.x == 0 && kind == kFusedHelp) {
+                if constexpr (REFINE) there_before = (s_seen[0] | s_seen[1] | s_seen[2] | s_seen[3]) != 0;
+                else there_before = !pair_missing(read_pair(fw.ends2(ti)));
+            }
+            if (threadIdx.x == 0 && fused_publishes(kind, there_before)) {
+                if constexpr (REFINE) {
+                    // x2 is there before the tile's words are, and so before any
+                    // x of the tile is stored
+                    if (kind == kFusedHelp) publish_pair(fw.x2(ti), xo[0], tile_end);
+                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                }
+                publish_ends(fw.ends4(ti), fw.ends2(ti), mine);
+            }
             BlockEnds e{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             float before = 0.0f, after = 0.0f;
             bool there;  // every block that this tile waits for
